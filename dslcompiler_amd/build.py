@@ -45,6 +45,7 @@ HIP_SOURCES = [
     CSRC / "kernels" / "mfma_tile.hip",
     CSRC / "kernels" / "swiglu_wide.hip",
     CSRC / "kernels" / "swiglu_decode.hip",
+    CSRC / "kernels" / "flex_tile.hip",
     CSRC / "kernels" / "pack.hip",
     CSRC / "llk_abi.cpp",  # host code that calls the HIP runtime
     CSRC / "kernel_fn.cpp",

@@ -10,3 +10,4 @@
 #include "swiglu_wide.hip"
 #include "pack.hip"
 #include "swiglu_decode.hip"
+#include "flex_tile.hip"

@@ -663,6 +663,15 @@ const char* split_reduce_symbol() {
   return name.c_str();
 }
 
+// The reduce of a k split's planes into y.
+template <int MODE, int OUT, bool YVEC>
+static hipError_t launch_reduce(const TileArgs& a, const llk::ModuleFns* mod, hipStream_t s) {
+  const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
+  return launch_kernel(mod, reinterpret_cast<const void*>(split_reduce_kernel<MODE, OUT, YVEC>),
+                       &split_reduce_symbol<MODE, OUT, YVEC>,
+                       dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a);
+}
+
 template <int MODE, int OUT, bool YVEC, bool SPLIT, bool RM = false>
 static hipError_t launch_tile_t(const TileArgs& a, const llk::ModuleFns* mod, hipStream_t s) {
   void (*fn)(TileArgs);
@@ -688,10 +697,7 @@ static hipError_t launch_split(const TileArgs& a, const llk::ModuleFns* mod, hip
   // Partials are fp32 planes with 16-byte aligned rows: one instantiation.
   hipError_t e = launch_tile_t<MODE, kOutF32, true, true, RM>(a, mod, s);
   if (e != hipSuccess) return e;
-  const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
-  return launch_kernel(mod, reinterpret_cast<const void*>(split_reduce_kernel<MODE, OUT, YVEC>),
-                       &split_reduce_symbol<MODE, OUT, YVEC>,
-                       dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a);
+  return launch_reduce<MODE, OUT, YVEC>(a, mod, s);
 }
 
 template <int MODE, int OUT, bool YVEC, bool RM = false>
@@ -773,6 +779,46 @@ hipError_t llk_launch_tile(int mode, const uint16_t* x, int64_t ldx, const void*
 #endif
 #if !defined(LLK_CO_OP) || LLK_CO_OP == 0
   if (mode == 0) return launch_mode<0>(a, out, yvec, mod, s);
+#endif
+  return hipErrorInvalidValue;
+}
+
+// Internal: sums the S planes part[s][mat][M][n_pad] (n_pad = 128 NB) that a
+// k split left, in split order, applies the epilogue of `mode` (1 SwiGLU, 0
+// GEMM, with accumulate y += sum) and stores y.
+hipError_t llk_launch_split_reduce(int mode, const void* part, int S, void* y, int64_t ldy, int M,
+                                   int N, int NB, int out, bool yvec, bool accumulate,
+                                   const llk::ModuleFns* mod, hipStream_t s) {
+  using namespace llk_gfx950;
+  if (part == nullptr || S < 1 || M < 1 || N < 1 || (accumulate && mode != 0))
+    return hipErrorInvalidValue;
+  TileArgs a{};
+  a.y = y;
+  a.ldy = ldy;
+  a.M = M;
+  a.N = N;
+  a.S = S;
+  a.n_pad = NB * 128;
+  a.part = static_cast<float*>(const_cast<void*>(part));
+  a.accumulate = accumulate ? 1 : 0;
+#if !defined(LLK_CO_OP) || LLK_CO_OP == 1
+  if (mode == 1 && out == kOutBF16)
+    return yvec ? launch_reduce<1, kOutBF16, true>(a, mod, s)
+                : launch_reduce<1, kOutBF16, false>(a, mod, s);
+  if (mode == 1 && out == kOutF32)
+    return yvec ? launch_reduce<1, kOutF32, true>(a, mod, s)
+                : launch_reduce<1, kOutF32, false>(a, mod, s);
+#endif
+#if !defined(LLK_CO_OP) || LLK_CO_OP == 0
+  if (mode == 0 && out == kOutBF16)
+    return yvec ? launch_reduce<0, kOutBF16, true>(a, mod, s)
+                : launch_reduce<0, kOutBF16, false>(a, mod, s);
+  if (mode == 0 && out == kOutF16)
+    return yvec ? launch_reduce<0, kOutF16, true>(a, mod, s)
+                : launch_reduce<0, kOutF16, false>(a, mod, s);
+  if (mode == 0 && out == kOutF32)
+    return yvec ? launch_reduce<0, kOutF32, true>(a, mod, s)
+                : launch_reduce<0, kOutF32, false>(a, mod, s);
 #endif
   return hipErrorInvalidValue;
 }

@@ -68,6 +68,14 @@ hipError_t llk_launch_tile_rowmajor(int mode, const uint16_t* x, int64_t ldx, co
                                     int64_t ldy, int M, int N, int K, int S, void* part, int out,
                                     bool yvec, bool accumulate, const llk::ModuleFns* mod,
                                     hipStream_t s);
+bool llk_flex_fits(int64_t M, int64_t K, int64_t ldx, int64_t ldw0, int64_t ldw1);
+hipError_t llk_launch_flex(int mode, int cfg, const uint16_t* x, int64_t ldx, const void* w0,
+                           int64_t ldw0, const void* w1, int64_t ldw1, void* y, int64_t ldy,
+                           int M, int N, int K, int S, void* part, int out, bool accumulate,
+                           bool rowmajor, const llk::ModuleFns* mod, hipStream_t s);
+hipError_t llk_launch_split_reduce(int mode, const void* part, int S, void* y, int64_t ldy, int M,
+                                   int N, int NB, int out, bool yvec, bool accumulate,
+                                   const llk::ModuleFns* mod, hipStream_t s);
 hipError_t llk_launch_pad_rows(const uint16_t* x, int64_t ldx, int M, int K, uint16_t* out,
                                int64_t ldo, const llk::ModuleFns* mod, hipStream_t s);
 hipError_t llk_launch_pack(const uint16_t* w, int64_t ld, int K, int N, int KB, int NB, void* out,
@@ -236,20 +244,23 @@ bool evict_one_workspace(DeviceState& st, const Workspace* keep) {
 // graph is pinned instead (the graph names it) and is never freed.  Growth
 // is geometric (x1.5 at least).  *held is the library workspace handed out
 // (null for a caller's scratch or when nothing is needed): the caller gives
-// it back with release_workspace after enqueuing its launches.
-int get_workspace(int dev, size_t need, llk_kernel_context* ctx, void** out, Workspace** held) {
+// it back with release_workspace after enqueuing its launches.  `asked`: what
+// a caller's scratch must hold (at least `need`).
+int get_workspace(int dev, size_t need, size_t asked, llk_kernel_context* ctx, void** out,
+                  Workspace** held) {
   *out = nullptr;
   *held = nullptr;
-  if (need == 0) return LLK_OK;
+  if (asked == 0) return LLK_OK;
   if (ctx && ctx->scratch) {
-    if (ctx->scratch_size < need)
+    if (ctx->scratch_size < asked)
       return fail(LLK_ERR_SCRATCH, "scratch_size %zu < required %zu bytes", ctx->scratch_size,
-                  need);
+                  asked);
     if (reinterpret_cast<uintptr_t>(ctx->scratch) % 256 != 0)
       return fail(LLK_ERR_SCRATCH, "scratch must be 256-byte aligned");
     *out = ctx->scratch;
     return LLK_OK;
   }
+  if (need == 0) return LLK_OK;
   DeviceState& st = g_dev[dev];
   const auto key = workspace_key(ctx ? static_cast<hipStream_t>(ctx->stream) : nullptr);
   std::lock_guard<std::mutex> lk(st.mu);
@@ -397,6 +408,8 @@ struct Plan {
   size_t ws_bytes = 0;   // workspace the plan needs
   bool too_large = false;  // tile path: K beyond the kernel's 32-bit offsets
   int64_t head_nb = 0;   // tile path: leading n-blocks launched unsplit (S applies to the rest)
+  int flex = 0;          // flex tile kernel: its tile (222, 224, 244); S as above
+  size_t flex_bytes = 0; // ... and the planes it needs; ws_bytes stays the other plan's
   int wide = 0;          // tile path, fused SwiGLU with bf16 output: the wide kernel's B
                          // (16 B columns per tile and matrix; 0 = the 128-column kernel)
 };
@@ -754,8 +767,8 @@ Plan plan_launch_base(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
 // at M = 128: the SwiGLU's 216 workgroups unsplit, the down projection's 40
 // in 6 splits); otherwise the tile kernels.  With X unknown (sizing), the
 // larger of the two workspaces.
-Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const llk_tensor2d* x,
-                 size_t max_ws = SIZE_MAX, bool accumulate = false, bool out_bf16 = true) {
+Plan plan_launch_large(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
+                       const llk_tensor2d* x, size_t max_ws, bool accumulate, bool out_bf16) {
   if (M > 64 && M <= std::min<int64_t>(256, llk::tunable("midm_max_m")) &&
       llk::tunable("decode_tile") != 0 && llk_decode_tile_fits((int)M, K, x ? x->stride0 : K)) {
     int64_t forced = llk::tunable("decode_splits");
@@ -781,6 +794,147 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
   return plan_launch_base(nmat, M, K, KB, NB, x, max_ws, accumulate, out_bf16);
 }
 
+// The flex tile kernel (kernels/flex_tile.hip) against the plan above it.
+// Both times are modelled in microseconds, fitted on MI355X measurements of
+// 370 random shapes (M 65..4097, K 512..13824, N 512..14336, both operations;
+// each model within 4-10% rms, the tile kernel's unsplit one 15%).  Over them
+// the choice the models make runs 1.42x the plan without this kernel in the
+// geometric mean; always taking the fastest measured would give 1.43x.
+//   us = a + b n kbs + c kbs + d (MB of Y, or of planes when S > 1)
+//          + e (MB of weights) + f n + g (MB of weights beyond 80)
+// with n = ceil(workgroups / 256) and kbs = 64-k steps per split: the
+// smaller tiles pay less for a short grid or a ragged edge, the larger ones
+// less per multiply-add.
+struct FlexModel {
+  int cfg, tm, tn;  // tile: rows, MFMA rows
+  double one[7], many[7];
+};
+constexpr FlexModel kFlex[] = {
+    {222, 64, 64, {2.87, 0.197, 0.044, 0.124, 0, 0.30, 0.117},
+     {6.3, 0.090, 0.162, 0.453, 0.0065, 0.69, 0.655}},
+    {224, 64, 128, {3.46, 0.283, 0.040, 0.169, 0.010, 0.29, 0.146},
+     {7.4, 0.177, 0.142, 0.324, 0.002, 0.75, 0.204}},
+    {244, 128, 128, {3.89, 0.402, 0, 0.192, 0.0076, 0.89, 0.166},
+     {9.5, 0.349, 0, 0.307, 0.021, 0, 0.146}},
+};
+
+// Modelled microseconds of a plan of the other kernels above 64 rows.
+double plan_us(const Plan& p, int nmat, int64_t M, int64_t KB, int64_t NB) {
+  const double y_mb = M * NB * 128 * 3e-6, w_mb = KB * NB * 16384e-6 * nmat;
+  const double past = std::max(0.0, w_mb - 80.0);
+  const int64_t kbs = (KB + p.S - 1) / p.S;
+  const double planes = p.S * nmat * M * NB * 512e-6;
+  auto rounds = [](int64_t wgs) { return (double)((wgs + 255) / 256); };
+  if (p.dtile) {
+    const double t = rounds((nmat == 2 ? NB * 2 : NB) * p.S) * kbs;
+    return p.S > 1 ? 7.2 + 0.529 * t + 0.668 * planes + 0.002 * w_mb + 0.043 * past
+                   : 4.0 + 0.516 * t + 0.269 * y_mb + 0.024 * w_mb;
+  }
+  const int64_t tm = (M + 255) / 256;
+  double us;
+  if (p.wide && p.S == 1) {
+    const double t = rounds(tm * ((NB * 8 + p.wide - 1) / p.wide)) * (kbs + 2) * p.wide / 8.0;
+    us = 3.2 + 1.22 * t + 0.266 * y_mb + 0.092 * past;
+  } else {
+    const int64_t per = nmat == 2 ? 1 : 2, tail = NB - p.head_nb;
+    const double t =
+        p.wide ? rounds(tm * ((NB * 8 + p.wide - 1) / p.wide) * p.S) * (kbs + 2) * p.wide / 8.0
+               : rounds(tm * ((tail + per - 1) / per) * p.S) * (kbs + 2);
+    const double part = (double)tail / NB;
+    us = p.S > 1 ? 13.4 + 1.044 * t + part * (0.208 * planes + 0.13 * past)
+                 : 1.8 + 1.096 * t + 0.356 * y_mb + 0.021 * w_mb + 0.033 * past;
+    if (p.head_nb > 0) us += 1.53 * rounds(tm * (p.head_nb / per)) * (KB + 2);
+  }
+  if (p.pad) us += 3.0 + M * KB * 256 / 3e6;  // the padded copy of X
+  return us;
+}
+
+// The plan: above 64 rows the flex tile kernel where it is modelled faster.
+// The choice depends on the shape and X's alignment alone -- not on the
+// result type or on the workspace at hand -- so a bf16 result stays the
+// rounding of the fp32 one.
+// Kept on the other kernels: 512 or fewer k, 768 or fewer for C += A B (the
+// launches and scratch of such plans are part of what callers and tests hold
+// this library to), X at an odd base or row stride (K itself a
+// multiple of 8) in fewer than 128 workgroups (the same), more
+// than 128 MB of weights (the k loop then streams from HBM; of ten shapes
+// measured there this kernel was 6 and 9% faster on two and 5 to 33% slower on
+// the others), X beyond one launch's 32-bit offsets, and every call for which a knob or a schedule
+// record has chosen among those kernels.  A caller's scratch (max_ws) that
+// holds the other plan but not this one's planes gets the other plan.
+Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const llk_tensor2d* x,
+                 size_t max_ws = SIZE_MAX, bool accumulate = false, bool out_bf16 = true) {
+  Plan p = plan_launch_large(nmat, M, K, KB, NB, x, max_ws, accumulate, out_bf16);
+  const int64_t knob = llk::tunable("flex_tile");
+  const int64_t forced_s = llk::tunable("tile_splits");
+  int cfg = 0;
+  int64_t S = 1;
+  if (knob > 1) {
+    cfg = (int)knob;
+    const int64_t kbs = (KB + std::max<int64_t>(1, forced_s) - 1) / std::max<int64_t>(1, forced_s);
+    S = (KB + kbs - 1) / kbs;
+  } else {
+    if (knob == 0 || M <= 64 || KB <= (accumulate ? 12 : 8) ||
+        KB * NB * nmat > 8192 || (p.chunk > 0 && p.chunk < M) || p.too_large || p.ws_bytes > max_ws || forced_s > 0 ||
+        llk::tunable("tile_wide") != 1 || llk::tunable("tile_wgs_per_wave") != 256 ||
+        llk::tunable("tile_tail_split") != 1 || llk::tunable("tile_min_kb") != 4 ||
+        llk::tunable("midm_max_m") != 128 || llk::tunable("decode_tile") != 1 ||
+        llk::tunable("decode_splits") > 0)
+      return p;
+    llk::ScheduleEntry se;
+    if (db_entry(nmat, M, &se) && se.grain_size > 0) return p;
+    const Plan ref = accumulate || !out_bf16 || max_ws != SIZE_MAX
+                         ? plan_launch_large(nmat, M, K, KB, NB, x, SIZE_MAX, false, true)
+                         : p;
+    // X rows that start inside a 128-byte line (whose lines are read twice)
+    // slow a step by 8%, rows off the 16 bytes by 20% and at odd elements by
+    // 25% (K = 1600 against 1599 and 1598, N = 4288, M = 3779: 60.8, 67.1 and
+    // 67.4 us with the larger tiles, 18.2 to 20.1 us at M = 400).
+    const bool aligned = x && x_vec_ok(x);
+    const double slow =
+        !x ? 1.0
+           : aligned ? (x->stride0 % 64 != 0 ? 1.08 : 1.0)
+                     : (x->stride0 | (int64_t)(reinterpret_cast<uintptr_t>(x->data) / 2)) & 1 ? 1.25
+                                                                                              : 1.20;
+    // taken when modelled 5% faster; 12% on rows off the 16 bytes, where the
+    // two models are rougher
+    double best = (aligned ? 0.95 : 0.88) * plan_us(ref, nmat, M, KB, NB);
+    if (!aligned && K % 8 == 0 && (M + 63) / 64 * (NB * 2 * nmat) < 128) return p;
+    const double y_mb = M * NB * 128 * 3e-6, w_mb = KB * NB * 16384e-6 * nmat;
+    for (const FlexModel& f : kFlex) {
+      const int64_t tiles = (M + f.tm - 1) / f.tm * (NB * 128 * nmat / f.tn);
+      if (tiles > 65536) continue;
+      for (const int64_t want : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        if (want > 1 && (tiles * want > 1024 || KB / want < 3)) break;
+        const int64_t kbs = (KB + want - 1) / want, s = (KB + kbs - 1) / kbs;
+        const double n = (double)((tiles * s + 255) / 256);
+        const double* c = s == 1 ? f.one : f.many;
+        const double us = c[0] + slow * c[1] * n * kbs + c[2] * kbs +
+                          c[3] * (s == 1 ? y_mb : s * nmat * M * NB * 512e-6) + c[4] * w_mb +
+                          c[5] * n + c[6] * std::max(0.0, w_mb - 80.0);
+        if (us < best) {
+          best = us;
+          cfg = f.cfg;
+          S = s;
+        }
+      }
+    }
+  }
+  if (!cfg || (x && !llk_flex_fits(M, K, x->stride0, 0, 0))) return p;
+  const size_t bytes = S > 1 ? (size_t)S * nmat * M * NB * 512 : 0;
+  if (bytes > max_ws) return p;
+  if (!x) {  // sizing: whichever needs more
+    p.ws_bytes = std::max(p.ws_bytes, bytes);
+    return p;
+  }
+  Plan q;
+  q.flex = cfg;
+  q.S = (int)S;
+  q.flex_bytes = bytes;
+  q.ws_bytes = std::max(p.ws_bytes, bytes);
+  return q;
+}
+
 // K == 0: the reference's verifiers accept an empty reduction
 // (LLKOps.cpp:42-83, 336-348) and its zero-filled fp32 accumulators
 // (FuseDoubleContraction.cpp:119-135) give SiLU(0) * 0 = +0 for SwiGLU and
@@ -804,18 +958,25 @@ int run_contraction(int mode, const llk_tensor2d* x, const llk_packed_weights* w
                     bool accumulate = false) {
   const int64_t M = x->dim0, K = x->dim1;
   const int nmat = mode == 1 ? 2 : 1;
-  const Plan p = plan_launch(nmat, M, K, w0->KB, w0->NB, x, max_ws, accumulate,
-                             out_dtype == LLK_BF16);
+  Plan p = plan_launch(nmat, M, K, w0->KB, w0->NB, x, max_ws, accumulate, out_dtype == LLK_BF16);
+  size_t asked = p.ws_bytes;
+  if (p.flex && ctx && ctx->scratch && ctx->scratch_size < p.ws_bytes) {
+    const Plan q = plan_launch_large(nmat, M, K, w0->KB, w0->NB, x, max_ws, accumulate,
+                                     out_dtype == LLK_BF16);
+    asked = q.ws_bytes;
+    if (ctx->scratch_size < p.flex_bytes) p = q;
+  }
   if (p.too_large)
     return fail(LLK_ERR_SHAPE, "%s: K=%lld too large for M=%lld (the tile kernel needs K <= %lld)",
                 what, (long long)K, (long long)M, (long long)(((int64_t)1 << 31) / 512 - 64));
-  if (p.ws_bytes > max_ws)
+  if ((p.flex ? p.flex_bytes : p.ws_bytes) > max_ws)
     return fail(LLK_ERR_SCRATCH,
                 "%s: M=%lld K=%lld needs %zu workspace bytes, more than the %zu available",
                 what, (long long)M, (long long)K, p.ws_bytes, max_ws);
   void* ws = nullptr;
   Workspace* held = nullptr;
-  int rc = get_workspace(dev, p.ws_bytes, ctx, &ws, &held);
+  int rc = get_workspace(dev, p.flex ? p.flex_bytes : p.ws_bytes, std::min(asked, max_ws), ctx, &ws,
+                         &held);
   if (rc) return rc;
   hipStream_t s = stream_of(ctx);
   BindDone bind(held, s);
@@ -834,6 +995,16 @@ int launch_contraction(int mode, const llk_tensor2d* x, const llk_packed_weights
   const int64_t M = x->dim0, K = x->dim1, N = w0->N;
   const bool yvec = y_vec_ok(y, out_dtype);
   hipError_t e = hipSuccess;
+  if (p.flex) {
+    e = llk_launch_flex(mode, p.flex, static_cast<const uint16_t*>(x->data), x->stride0, w0->dev, 0,
+                        w1 ? w1->dev : nullptr, 0, y->data, y->stride0, (int)M, (int)N, (int)K, p.S,
+                        body, out_dtype, accumulate, false, mod, s);
+    if (e == hipSuccess && p.S > 1)
+      e = llk_launch_split_reduce(mode, body, p.S, y->data, y->stride0, (int)M, (int)N, (int)w0->NB,
+                                  out_dtype, yvec, accumulate, mod, s);
+    if (e != hipSuccess) return fail_hip(e, what);
+    return LLK_OK;
+  }
   if (p.dtile) {
     e = llk_launch_decode_tile(mode, static_cast<const uint16_t*>(x->data), x->stride0, w0->dev,
                                w1 ? w1->dev : nullptr, y->data, y->stride0, (int)M, (int)N,
@@ -1319,6 +1490,15 @@ int llk_describe_launch(int operation, int64_t M, int64_t N, int64_t K, unsigned
                 (long long)K, (long long)M, (long long)(((int64_t)1 << 31) / 512 - 64));
   out->splits = p.S;
   out->workspace_bytes = p.ws_bytes;
+  if (p.flex) {
+    const int64_t tm = p.flex == 244 ? 128 : 64, cols = (p.flex == 222 ? 64 : 128) / nmat;
+    out->kernel = 4;
+    out->tile_columns = cols;
+    out->workgroups = (M + tm - 1) / tm * ((N + cols - 1) / cols) * p.S;
+    out->threads_per_workgroup = 256;
+    out->launches = p.S > 1 ? 2 : 1;
+    return LLK_OK;
+  }
   if (p.dtile) {
     out->kernel = 3;
     out->group_width = 0;
@@ -1587,9 +1767,13 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   };
   int S = p.S;
   size_t ws_bytes = p.ws_bytes;
+  size_t asked = p.ws_bytes;
   bool tile = false;
   int64_t head_cols = 0;  // tile form: columns of the unsplit head launch
-  if (p.dtile && M <= 128) {
+  if (p.flex) {  // row-major weights of any alignment
+    if (!llk_flex_fits(M, K, x->stride0, wg->stride0, mode == 1 ? wu->stride0 : 0)) return LLK_OK;
+    ws_bytes = p.flex_bytes;
+  } else if (p.dtile && M <= 128) {
     if (!fits(&llk_decode_rowmajor_fits)) return LLK_OK;
   } else if (!p.skinny && mode == 1 && (out_dtype == LLK_BF16 || out_dtype == LLK_FP32) &&
              !accumulate && !p.pad && p.chunk >= M && fits(&llk_tile_rowmajor_fits)) {
@@ -1612,7 +1796,8 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   if (rc) return rc;
   void* ws = nullptr;
   Workspace* held = nullptr;
-  if ((rc = get_workspace(dev, ws_bytes, ctx, &ws, &held))) return rc;
+  if (!p.flex) asked = ws_bytes;
+  if ((rc = get_workspace(dev, ws_bytes, asked, ctx, &ws, &held))) return rc;
   *taken = true;
   hipStream_t s = stream_of(ctx);
   BindDone bind(held, s);
@@ -1620,7 +1805,14 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   const uint16_t* const wgd = static_cast<const uint16_t*>(wg->data);
   const uint16_t* const wud = mode == 1 ? static_cast<const uint16_t*>(wu->data) : nullptr;
   hipError_t e = hipSuccess;
-  if (tile) {
+  if (p.flex) {
+    e = llk_launch_flex(mode, p.flex, xd, x->stride0, wgd, wg->stride0, wud,
+                        mode == 1 ? wu->stride0 : 0, y->data, y->stride0, (int)M, (int)N, (int)K, S,
+                        ws, out_dtype, accumulate, true, mod, s);
+    if (e == hipSuccess && S > 1)
+      e = llk_launch_split_reduce(mode, ws, S, y->data, y->stride0, (int)M, (int)N, (int)NB,
+                                  out_dtype, y_vec_ok(y, out_dtype), accumulate, mod, s);
+  } else if (tile) {
     // head columns unsplit, then the rest with the plan's splits (offsets of
     // 128-column multiples keep every row 16-byte aligned)
     const bool yv = y_vec_ok(y, out_dtype);
@@ -1644,7 +1836,8 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   bind.end();
   release_workspace(dev, held, s, bind.bound());
   return e == hipSuccess ? LLK_OK
-                         : fail_hip(e, tile ? "tile kernel (row-major weights)"
+                         : fail_hip(e, p.flex ? "flex tile kernel (row-major weights)"
+                                       : tile ? "tile kernel (row-major weights)"
                                             : "decode tile kernel (row-major weights)");
 }
 

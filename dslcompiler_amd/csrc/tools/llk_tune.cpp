@@ -155,7 +155,7 @@ int main(int argc, char** argv) {
   cands.swap(uniq);
   std::printf("M=%lld (bucket %d) N=%lld K=%lld op=%s kernel=%s\n", (long long)M, bucket,
               (long long)N, (long long)K, op.c_str(),
-              small ? "small_m" : midm ? "decode_tile (mid M)" : "mfma_tile");
+              small ? "small_m" : midm ? "decode_tile (mid M)" : own.kernel == 4 ? "flex_tile" : "mfma_tile");
   std::printf("Generated %zu candidate launches\n", cands.size());
 
   if (!dry) {
@@ -257,6 +257,7 @@ int main(int argc, char** argv) {
     // BM: rows per workgroup (the decode tile kernel: 64, or 128 / 256 at mid M)
     const int64_t BM = c.plan.kernel == 0   ? (M <= 32 ? 32 : 64)
                        : c.plan.kernel == 3 ? (M <= 64 ? 64 : M <= 128 ? 128 : 256)
+                       : c.plan.kernel == 4 ? (c.plan.tile_columns * nmat == 64 ? 64 : 128)
                                             : 256;
     // BN 0 / grain_size 0: the dispatcher chooses for each shape (for M <= 64
     // the decode tile kernel where it applies, else the small-M kernel's

@@ -129,6 +129,25 @@ def predict(op: str, M: int, N: int, K: int, machine_path: str = str(MACHINE)) -
         # the split reduce: its own pass after the main kernel
         reduce = cal["decode_tile_reduce_s"] if S > 1 else 0.0
         t = max(compute, memory, per_cu, cal["launch_min_s"]) + reduce + gap
+    elif plan["kernel"] == "flex_tile":
+        # 64 or 128 rows by 64 or 128 MFMA rows per workgroup: a fixed time
+        # per 64-k step and round of workgroups, whatever holds it (LDS and
+        # the load path, not the MFMAs)
+        mrows = plan["tile_columns"] * nmat
+        rows = 64
+        if mrows == 128 and plan["workgroups"] // S < math.ceil(M / 64) * math.ceil(
+                N / plan["tile_columns"]):
+            rows = 128
+        kbs = math.ceil(math.ceil(K / 64) / S)
+        step = cal[f"flex_step_{rows}x{mrows}_s"]
+        per_cu = 2.0 * cal["decode_tile_fill_s"] + math.ceil(plan["workgroups"] / cus) * kbs * step
+        compute = math.ceil(plan["workgroups"] / cus) * kbs * 2.0 * rows * mrows * 64 / (
+            cal["small_m_flops_per_cu"])
+        partials = 2.0 * 4.0 * S * nmat * M * N if S > 1 else 0.0
+        nbytes = 2.0 * nmat * K * N + 2.0 * M * K + 2.0 * M * N + partials
+        memory = nbytes / cal["decode_tile_stream_bytes_per_s"]
+        reduce = cal["decode_tile_reduce_s"] if S > 1 else 0.0
+        t = max(compute, memory, per_cu, cal["launch_min_s"]) + reduce + gap
     else:
         groups = plan["workgroups"]
         mrows = 32 * math.ceil(M / 32)
