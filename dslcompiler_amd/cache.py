@@ -87,7 +87,8 @@ def memref(t) -> MemRef2D:
     else:
         if t.dim() != 2:
             raise ValueError("memref operands are 2-D")
-        ptr, (d0, d1), (s0, s1) = t.data_ptr(), t.shape, t.stride()
+        ptr = t.data_ptr()
+        return MemRef2D(ptr, ptr, 0, *t.shape, *t.stride())
     return MemRef2D(ptr, ptr, 0, d0, d1, s0, s1)
 
 
@@ -116,10 +117,10 @@ class KernelFn:
     def __call__(self, x, wg, wu, init, result) -> None:
         """Operands: 2-D torch tensors or numpy arrays (wu None for a
         matmul entry); raises LLKError on a failed call."""
-        m = [memref(t) if t is not None else None for t in (x, wg, wu, init, result)]
-        if result is init:
-            m[4] = m[3]
-        self._fn(*(C.byref(v) if v is not None else None for v in m))
+        i = memref(init) if init is not None else None
+        r = i if result is init else memref(result) if result is not None else None
+        self._fn(memref(x) if x is not None else None, memref(wg) if wg is not None else None,
+                 memref(wu) if wu is not None else None, i, r)
         _check_kernel_fn()
 
 

@@ -107,7 +107,6 @@ constexpr int kMaxDevices = 64;
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
-  hipEvent_t done = nullptr;  // completes after the last call that used it (see bind)
   bool pinned = false;        // used under graph capture: a graph may name it, never freed
   int busy = 0;               // calls between get_workspace and release_workspace
   uint64_t tick = 0;          // last use, for LRU eviction
@@ -201,18 +200,19 @@ std::pair<uintptr_t, uint64_t> workspace_key(hipStream_t s) {
   return {reinterpret_cast<uintptr_t>(s), s == hipStreamPerThread ? thread_id : 0};
 }
 
-// Frees a library workspace's buffer once the last call that used it has
-// finished on the GPU (its `done` event; a workspace never used yet has
-// none).  Called with the device mutex held, for idle, unpinned entries.
-void free_workspace_buffer(Workspace* w) {
-  if (w->done) (void)hipEventSynchronize(w->done);
-  if (w->ptr) (void)hipFree(w->ptr);
-  w->ptr = nullptr;
-  w->bytes = 0;
+// Whether `s` is capturing a graph (or that cannot be told).
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  const bool yes = hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+  if (yes) (void)hipGetLastError();  // a failed query leaves no error for the next call
+  return yes;
 }
 
 // Evicts the least recently used idle, unpinned workspace of `st` other
-// than `keep`; false if there is none.
+// than `keep`; false if there is none, or if the device cannot be waited for
+// (a graph is being captured).  Its stream may be gone, with work still
+// queued, so the whole device is waited for: eviction is rare.  Called with
+// the device mutex held.
 bool evict_one_workspace(DeviceState& st, const Workspace* keep) {
   auto victim = st.ws.end();
   for (auto it = st.ws.begin(); it != st.ws.end(); ++it) {
@@ -221,8 +221,13 @@ bool evict_one_workspace(DeviceState& st, const Workspace* keep) {
     if (victim == st.ws.end() || w.tick < victim->second.tick) victim = it;
   }
   if (victim == st.ws.end()) return false;
-  free_workspace_buffer(&victim->second);
-  if (victim->second.done) (void)hipEventDestroy(victim->second.done);
+  if (victim->second.ptr) {
+    if (hipDeviceSynchronize() != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    (void)hipFree(victim->second.ptr);
+  }
   st.ws.erase(victim);
   return true;
 }
@@ -235,17 +240,17 @@ bool evict_one_workspace(DeviceState& st, const Workspace* keep) {
 // on the capture stream is the caller's race, as with any captured buffer.)
 // The library keeps at most `max_workspaces` of them per device (tunable,
 // default 16): a new stream (or thread, on the per-thread default stream)
-// beyond that evicts the least recently used idle one.  A buffer is freed
-// (on eviction, on growth, or by llk_workspace_trim) only after its event,
-// which completes with the last kernel of the last call that used it, has
-// completed (BindDone: the event rides on the launches themselves), so work still
-// queued on a stream -- even one destroyed since -- never loses its
-// buffer; a workspace that a call used while its stream was capturing a
-// graph is pinned instead (the graph names it) and is never freed.  Growth
-// is geometric (x1.5 at least).  *held is the library workspace handed out
-// (null for a caller's scratch or when nothing is needed): the caller gives
-// it back with release_workspace after enqueuing its launches.  `asked`: what
-// a caller's scratch must hold (at least `need`).
+// beyond that evicts the least recently used idle one.  A buffer is freed on
+// growth only after its stream, and on eviction or by llk_workspace_trim only
+// after the device, has been waited for, so work still queued -- even on a
+// stream destroyed since -- never loses its buffer, and no call pays for an
+// event of its own (naming one as a kernel's stop event cost 4 us a launch on
+// the host: two launches 11.6 -> 6 us).  A workspace that a call used while its
+// stream was capturing a graph is pinned instead (the graph names it) and is
+// never freed.  Growth is geometric (x1.5 at least).  *held is the library
+// workspace handed out (null for a caller's scratch or when nothing is
+// needed): the caller gives it back with release_workspace after enqueuing
+// its launches.  `asked`: what a caller's scratch must hold (at least `need`).
 int get_workspace(int dev, size_t need, size_t asked, llk_kernel_context* ctx, void** out,
                   Workspace** held) {
   *out = nullptr;
@@ -265,8 +270,7 @@ int get_workspace(int dev, size_t need, size_t asked, llk_kernel_context* ctx, v
   const auto key = workspace_key(ctx ? static_cast<hipStream_t>(ctx->stream) : nullptr);
   std::lock_guard<std::mutex> lk(st.mu);
   Workspace* w = nullptr;
-  const bool fresh_key = st.ws.find(key) == st.ws.end();
-  if (fresh_key) {
+  if (st.ws.find(key) == st.ws.end()) {
     const size_t cap = (size_t)std::max<int64_t>(1, llk::tunable("max_workspaces"));
     while (st.ws.size() >= cap && evict_one_workspace(st, nullptr)) {
     }
@@ -276,23 +280,19 @@ int get_workspace(int dev, size_t need, size_t asked, llk_kernel_context* ctx, v
   } catch (const std::bad_alloc&) {
     return fail(LLK_ERR_OUT_OF_MEMORY, "workspace bookkeeping");
   }
-  if (!w->done) {
-    const hipError_t e = hipEventCreateWithFlags(&w->done, hipEventDisableTiming);
-    if (e != hipSuccess) {
-      w->done = nullptr;
-      if (fresh_key) st.ws.erase(key);
-      return fail_hip(e, "hipEventCreate(workspace)");
-    }
-  }
   if (w->bytes < need) {
     const size_t bytes = std::max({need, w->bytes + w->bytes / 2, (size_t)1 << 20});
-    if (w->ptr && !w->pinned && w->busy == 0) {
-      free_workspace_buffer(w);  // this stream's earlier calls have finished with it
-    } else if (w->ptr) {
-      try {
-        st.retired.push_back(w->ptr);  // a graph or a concurrent call may still name it
-      } catch (const std::bad_alloc&) {
-        return fail(LLK_ERR_OUT_OF_MEMORY, "workspace bookkeeping");
+    if (w->ptr) {
+      const hipStream_t s = ctx ? static_cast<hipStream_t>(ctx->stream) : nullptr;
+      if (!w->pinned && w->busy == 0 && !capturing(s) && hipStreamSynchronize(s) == hipSuccess) {
+        (void)hipFree(w->ptr);  // this stream's earlier calls have finished with it
+      } else {
+        (void)hipGetLastError();
+        try {
+          st.retired.push_back(w->ptr);  // a graph or a concurrent call may still name it
+        } catch (const std::bad_alloc&) {
+          return fail(LLK_ERR_OUT_OF_MEMORY, "workspace bookkeeping");
+        }
       }
       w->ptr = nullptr;
       w->bytes = 0;
@@ -319,45 +319,13 @@ int get_workspace(int dev, size_t need, size_t asked, llk_kernel_context* ctx, v
   return LLK_OK;
 }
 
-// Binds a held workspace's `done` event to the calling thread's launches
-// from construction to end(): launch_kernel names it as each kernel's stop
-// event, so it completes with the call's last kernel.  Not when `s` is
-// capturing a graph (an event under capture would be a graph node, not a
-// point the host can wait for): release_workspace then pins the workspace.
-class BindDone {
- public:
-  BindDone(Workspace* w, hipStream_t s) : prev_(llk_gfx950::t_launch_done) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (w && hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
-      llk_gfx950::t_launch_done = w->done;
-      bound_ = true;
-    }
-  }
-  ~BindDone() { end(); }
-  void end() { llk_gfx950::t_launch_done = prev_; }
-  bool bound() const { return bound_; }
-  BindDone(const BindDone&) = delete;
-  BindDone& operator=(const BindDone&) = delete;
-
- private:
-  hipEvent_t prev_;
-  bool bound_ = false;
-};
-
 // Gives back a workspace from get_workspace once the call's launches are
-// enqueued on `s`.  `bound`: its `done` event rode on those launches
-// (BindDone); otherwise it is recorded on `s` now, or the workspace is
-// pinned when `s` is capturing a graph.
-void release_workspace(int dev, Workspace* w, hipStream_t s, bool bound = false) {
+// enqueued on `s`: pinned from then on when `s` is capturing a graph, whose
+// replays name the buffer.
+void release_workspace(int dev, Workspace* w, hipStream_t s) {
   if (!w) return;
+  const bool pin = capturing(s);
   DeviceState& st = g_dev[dev];
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  // Pinned too when the capture state or the record cannot be had: no event
-  // then marks this call's end, so the buffer must outlive it.
-  bool pin = !bound &&
-             (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
-  if (!bound && !pin && hipEventRecord(w->done, s) != hipSuccess) pin = true;
-  if (pin) (void)hipGetLastError();  // a failed query leaves no error for the next call
   std::lock_guard<std::mutex> lk(st.mu);
   if (pin) w->pinned = true;
   --w->busy;
@@ -979,11 +947,9 @@ int run_contraction(int mode, const llk_tensor2d* x, const llk_packed_weights* w
                          &held);
   if (rc) return rc;
   hipStream_t s = stream_of(ctx);
-  BindDone bind(held, s);
   rc = launch_contraction(mode, x, w0, w1, y, out_dtype, p, static_cast<uint8_t*>(ws), s, what,
                           mod, accumulate);
-  bind.end();
-  release_workspace(dev, held, s, bind.bound());
+  release_workspace(dev, held, s);
   return rc;
 }
 
@@ -1800,7 +1766,6 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   if ((rc = get_workspace(dev, ws_bytes, asked, ctx, &ws, &held))) return rc;
   *taken = true;
   hipStream_t s = stream_of(ctx);
-  BindDone bind(held, s);
   const uint16_t* const xd = static_cast<const uint16_t*>(x->data);
   const uint16_t* const wgd = static_cast<const uint16_t*>(wg->data);
   const uint16_t* const wud = mode == 1 ? static_cast<const uint16_t*>(wu->data) : nullptr;
@@ -1833,8 +1798,7 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
                                    (int)K, S, ws, out_dtype, y_vec_ok(y, out_dtype), accumulate,
                                    mod, s);
   }
-  bind.end();
-  release_workspace(dev, held, s, bind.bound());
+  release_workspace(dev, held, s);
   return e == hipSuccess ? LLK_OK
                          : fail_hip(e, p.flex ? "flex tile kernel (row-major weights)"
                                        : tile ? "tile kernel (row-major weights)"

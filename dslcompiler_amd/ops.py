@@ -23,25 +23,34 @@ from ._lib import (LLK_BF16, LLK_FP32, LLK_PACK_HOST_ONLY, LLK_PACK_KEEP_HOST, K
                    check, lib, tensor2d)
 
 
+_TORCH = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _TORCH
+    if _TORCH is None:
+        import torch
+        _TORCH = torch
+    return _TORCH
 
 
 def _stream_handle(stream=None) -> int:
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    if stream is None:
+        # the handle itself, without a Stream object around it (2.7 -> 0.1 us)
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:
+            return raw(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
+    return int(stream.cuda_stream)
 
 
 def _ctx(stream=None, scratch=None) -> KernelContext:
-    if scratch is not None:
-        _check_scratch(scratch)
-    ctx = KernelContext(None, 0, _stream_handle(stream))
-    if scratch is not None:
-        ctx.scratch = scratch.data_ptr()
-        ctx.scratch_size = scratch.numel() * scratch.element_size()
-    return ctx
+    if scratch is None:
+        return KernelContext(None, 0, _stream_handle(stream))
+    _check_scratch(scratch)
+    return KernelContext(scratch.data_ptr(), scratch.numel() * scratch.element_size(),
+                         _stream_handle(stream))
 
 
 def _check_scratch(t) -> None:
@@ -62,7 +71,7 @@ def _check_operand(t, name: str, dtypes) -> None:
     current CUDA device: the C ABI takes raw pointers and cannot tell host
     memory (a GPU memory fault when a kernel reads it) or another device's
     memory from the current device's."""
-    torch = _torch()
+    torch = _TORCH or _torch()
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise ValueError(f"{name} must be a CUDA tensor")
     if t.dtype not in dtypes:
@@ -75,7 +84,7 @@ def _check_operand(t, name: str, dtypes) -> None:
 def _t2d(t) -> _lib.Tensor2D:
     if t.dim() != 2:
         raise ValueError("expected a 2-D tensor")
-    return tensor2d(t.data_ptr(), t.shape[0], t.shape[1], t.stride(0), t.stride(1))
+    return _lib.Tensor2D(t.data_ptr(), *t.shape, *t.stride())
 
 
 def _out_dtype_code(dtype) -> int:
@@ -98,6 +107,7 @@ class PackedWeights:
 
     def __init__(self, handle: int, owned: bool = True):
         self._h = C.c_void_p(handle)
+        self._n = None  # N, once asked for (a handle's shape is fixed)
         self._owned = owned  # False: borrowed from a cache, never freed here
 
     # -- construction -------------------------------------------------------
@@ -196,7 +206,10 @@ class PackedWeights:
 
     @property
     def N(self) -> int:
-        return lib().llk_packed_weights_n(self.handle)
+        handle = self.handle
+        if self._n is None:
+            self._n = lib().llk_packed_weights_n(handle)
+        return self._n
 
     @property
     def K(self) -> int:
@@ -238,16 +251,24 @@ def pack_device_layout(w: np.ndarray) -> np.ndarray:
     return out
 
 
+def _result(x, n: int, dtype):
+    """An uninitialised [rows of x, n] result beside x."""
+    return x.new_empty((x.shape[0], n), dtype=dtype)
+
+
 def fused_swiglu(x, wg: PackedWeights, wu: PackedWeights, out=None, out_dtype=None,
                  stream=None, scratch=None):
     """Y = SiLU(X Wg) * (X Wu) on the current device (asynchronous)."""
     torch = _torch()
     _check_operand(x, "x", (torch.bfloat16,))
     if out is None:
-        out = torch.empty((x.shape[0], wg.N), dtype=out_dtype or torch.bfloat16, device=x.device)
-    _check_operand(out, "out", (torch.bfloat16, torch.float32))
-    check(lib().llk_swiglu_bf16(C.byref(_t2d(x)), wg.handle, wu.handle, C.byref(_t2d(out)),
-                                _out_dtype_code(out.dtype), C.byref(_ctx(stream, scratch))))
+        out = _result(x, wg.N, out_dtype or torch.bfloat16)
+        if out.dtype not in (torch.bfloat16, torch.float32):
+            _check_operand(out, "out", (torch.bfloat16, torch.float32))
+    else:
+        _check_operand(out, "out", (torch.bfloat16, torch.float32))
+    check(lib().llk_swiglu_bf16(_t2d(x), wg.handle, wu.handle, _t2d(out),
+                                _out_dtype_code(out.dtype), _ctx(stream, scratch)))
     return out
 
 
@@ -261,11 +282,13 @@ def matmul(a, b: PackedWeights, out=None, out_dtype=None, stream=None, scratch=N
     if out is None:
         if accumulate:
             raise ValueError("accumulate=True needs `out`, the accumulator")
-        out = torch.empty((a.shape[0], b.N), dtype=out_dtype or torch.float32, device=a.device)
-    _check_operand(out, "out", (torch.bfloat16, torch.float16, torch.float32))
+        out = _result(a, b.N, out_dtype or torch.float32)
+        if out.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+            _check_operand(out, "out", (torch.bfloat16, torch.float16, torch.float32))
+    else:
+        _check_operand(out, "out", (torch.bfloat16, torch.float16, torch.float32))
     fn = lib().llk_gemm_bf16_accumulate if accumulate else lib().llk_gemm_bf16
-    check(fn(C.byref(_t2d(a)), b.handle, C.byref(_t2d(out)), _out_dtype_code(out.dtype),
-             C.byref(_ctx(stream, scratch))))
+    check(fn(_t2d(a), b.handle, _t2d(out), _out_dtype_code(out.dtype), _ctx(stream, scratch)))
     return out
 
 
@@ -273,15 +296,18 @@ def mlp(x, wg: PackedWeights, wu: PackedWeights, wd: PackedWeights, y=None, z=No
         stream=None, scratch=None):
     """Y = SwiGLU(X) (bf16), Z = Y Wd (bf16); returns (y, z)."""
     torch = _torch()
-    _check_operand(x, "x", (torch.bfloat16,))
+    bf16 = torch.bfloat16
+    _check_operand(x, "x", (bf16,))
     if y is None:
-        y = torch.empty((x.shape[0], wg.N), dtype=torch.bfloat16, device=x.device)
+        y = _result(x, wg.N, bf16)
+    else:
+        _check_operand(y, "y", (bf16,))
     if z is None:
-        z = torch.empty((x.shape[0], wd.N), dtype=torch.bfloat16, device=x.device)
-    _check_operand(y, "y", (torch.bfloat16,))
-    _check_operand(z, "z", (torch.bfloat16,))
-    check(lib().llk_mlp_bf16(C.byref(_t2d(x)), wg.handle, wu.handle, wd.handle,
-                             C.byref(_t2d(y)), C.byref(_t2d(z)), C.byref(_ctx(stream, scratch))))
+        z = _result(x, wd.N, bf16)
+    else:
+        _check_operand(z, "z", (bf16,))
+    check(lib().llk_mlp_bf16(_t2d(x), wg.handle, wu.handle, wd.handle, _t2d(y), _t2d(z),
+                             _ctx(stream, scratch)))
     return y, z
 
 
