@@ -111,6 +111,24 @@ __device__ __forceinline__ int xcd_remap(int bid, int total) {
   return xcd * base + (xcd < extra ? xcd : extra) + local;
 }
 
+// 16 bytes at any 2-byte aligned address: one load or store, which the
+// hardware takes at any alignment of global memory.
+__device__ __forceinline__ u32x4 load16_any(const void* p) {
+  u32x4 v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
+  return v;
+}
+__device__ __forceinline__ void store16_any(void* p, const u32x4& v) {
+  __builtin_memcpy(__builtin_assume_aligned(p, 2), &v, 16);
+}
+// `n` (0..8) 16-bit elements at p, zeros after them.
+__device__ __forceinline__ u32x4 load16_part(const uint16_t* p, int n) {
+  uint32_t e[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) e[q] = q < n ? p[q] : 0u;
+  return u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+}
+
 // Output element types (values of llk_dtype).
 constexpr int kOutBF16 = 0, kOutF16 = 1, kOutF32 = 2;
 

@@ -78,15 +78,12 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const uint16_t* __restric
   if (idx >= (int64_t)M * per_row) return;
   const int64_t m = idx / per_row;
   const int c0 = (int)(idx % per_row) * 8;
-  uint16_t e[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) e[t] = (c0 + t < K) ? x[m * ldx + c0 + t] : (uint16_t)0;
-  uint4 v;
-  v.x = e[0] | ((uint32_t)e[1] << 16);
-  v.y = e[2] | ((uint32_t)e[3] << 16);
-  v.z = e[4] | ((uint32_t)e[5] << 16);
-  v.w = e[6] | ((uint32_t)e[7] << 16);
-  *reinterpret_cast<uint4*>(out + m * ldo + c0) = v;
+  // one load of any alignment (eight element loads before); the chunk K ends
+  // in by its elements
+  const uint16_t* const src = x + m * ldx + c0;
+  const llk_gfx950::u32x4 v = c0 + 8 <= K ? llk_gfx950::load16_any(src)
+                              : llk_gfx950::load16_part(src, c0 < K ? K - c0 : 0);
+  *reinterpret_cast<llk_gfx950::u32x4*>(out + m * ldo + c0) = v;
 }
 
 static const char* pad_rows_symbol() { return "_Z15pad_rows_kernelPKtliiPtl"; }

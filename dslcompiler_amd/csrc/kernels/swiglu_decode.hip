@@ -37,6 +37,12 @@ struct SkinnyArgs {
   bool accumulate;  // GEMM only: y += x w (the existing y read in its type)
 };
 
+// XVEC: rows 16-byte aligned and K a multiple of 8, so a chunk is wholly in or
+// out of a row.  Otherwise rows start at any element: one load of any alignment
+// per chunk, and the chunk K ends in by its elements.  (Eight element loads a
+// chunk set the kernel's pace, not the weights: SwiGLU M = 41, K = 2241, N =
+// 8496 51.0 -> 37.0 us, M = 30, K = 1091, N = 10128 30.0 -> 18.9 us, GEMM M = 3,
+// K = 3350, N = 4192 19.2 -> 10.6 us.)
 template <int MT, bool XVEC>
 __device__ __forceinline__ void load_x_frags(const SkinnyArgs& a, int kb, int lane,
                                              bf16x8 (&xf)[4][MT]) {
@@ -46,22 +52,16 @@ __device__ __forceinline__ void load_x_frags(const SkinnyArgs& a, int kb, int la
     for (int t = 0; t < MT; ++t) {
       const int m = t * 32 + (lane & 31);
       const int kk = kb * 64 + kq * 16 + (lane >> 5) * 8;
-      uint4 v = make_uint4(0, 0, 0, 0);
+      u32x4 v = {0, 0, 0, 0};
       if (m < a.M) {
         const uint16_t* src = a.x + (size_t)m * a.ldx + kk;
         if (XVEC) {
-          if (kk + 8 <= a.K) v = *reinterpret_cast<const uint4*>(src);
+          if (kk + 8 <= a.K) v = *reinterpret_cast<const u32x4*>(src);
         } else {
-          uint16_t e[8];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) e[q] = (kk + q < a.K) ? src[q] : (uint16_t)0;
-          v.x = e[0] | ((uint32_t)e[1] << 16);
-          v.y = e[2] | ((uint32_t)e[3] << 16);
-          v.z = e[4] | ((uint32_t)e[5] << 16);
-          v.w = e[6] | ((uint32_t)e[7] << 16);
+          v = kk + 8 <= a.K ? load16_any(src) : load16_part(src, a.K - kk);
         }
       }
-      xf[kq][t] = *reinterpret_cast<bf16x8*>(&v);
+      xf[kq][t] = __builtin_bit_cast(bf16x8, v);
     }
 }
 
