@@ -377,7 +377,7 @@ struct Plan {
   bool too_large = false;  // tile path: K beyond the kernel's 32-bit offsets
   int64_t head_nb = 0;   // tile path: leading n-blocks launched unsplit (S applies to the rest)
   int flex = 0;          // flex tile kernel: its tile (222, 224, 244); S as above
-  size_t flex_bytes = 0; // ... and the planes it needs; ws_bytes stays the other plan's
+  size_t need = 0;       // workspace the launches use; ws_bytes: what a caller's scratch holds
   int wide = 0;          // tile path, fused SwiGLU with bf16 output: the wide kernel's B
                          // (16 B columns per tile and matrix; 0 = the 128-column kernel)
 };
@@ -817,6 +817,110 @@ double plan_us(const Plan& p, int nmat, int64_t M, int64_t KB, int64_t NB) {
   return us;
 }
 
+// Up to 64 rows, one launch instead of the decode tile kernel's (or the small-M
+// kernel's) k split and reduce, or the small-M kernel's for K inside a 64-k step:
+// the small-M kernel unsplit at width 1 or 2, whose waves split k inside a
+// workgroup, or the flex tile kernel's 64-row tiles.  Microseconds, fitted on
+// 420 random shapes (M 1..64, K 512..13824, N 512..14336) within 4-7% rms, the
+// decode tile kernel 10%:
+//   small-M      c0 + c1 s + c2 W/2 r kbs + c3 r + c4 (MB of weights)
+//                  + (c5, X aligned, or c6) r kbs X + S > 1: c7 + c8 (MB of planes)
+//   decode tile  c0 + c1 r kbs + c3 (MB of weights) + c4 (MB beyond 80)
+//                  + S > 1: c5 + c6 (MB of planes)
+// with r = ceil(workgroups / 256), kbs = 64-k steps per split, s = steps per
+// wave and X = M / 32 times the wave groups that read it.  A second launch costs
+// the host too: 1 us.  Over the 296 shapes with N > 2176 the choice is 1.11x
+// the plan without it in the geometric mean of device time; M x N x K: GEMM
+// 2 x 2648 x 640 6.8 -> 3.9 us, 56 x 8560 x 4035 41.4 -> 23.7 us, SwiGLU
+// 60 x 5389 x 961 19.3 -> 9.3 us, 2 x 7163 x 1920 13.2 -> 11.4 us; none lost.
+struct SmallModel {
+  int nmat, mt, width;
+  double c[9];
+};
+constexpr SmallModel kSmall[] = {
+    {1, 1, 1, {2.28, 0.218, 0.138, 0, 0.058, 0.079, 0.272, 2.25, 0.261}},
+    {1, 1, 2, {1.82, 0.142, 0.147, 1.07, 0.043, 0.117, 0.303, 2.14, 0.422}},
+    {1, 2, 1, {2.68, 0.065, 0.127, 0.09, 0.046, 0.143, 0.312, 2.15, 0.287}},
+    {1, 2, 2, {3.90, 0.067, 0.193, 0.10, 0.054, 0.091, 0.261, 1.96, 0.245}},
+    {2, 1, 1, {2.19, 0.050, 0.305, 0.67, 0.063, 0.087, 0.270, 2.28, 0.128}},
+    {2, 1, 2, {1.75, 0.015, 0.303, 1.11, 0.046, 0.091, 0.270, 2.27, 0.214}},
+    {2, 2, 1, {2.47, 0.264, 0.257, 0.80, 0.079, 0.101, 0.278, 1.92, 0.317}},
+    {2, 2, 2, {2.37, 0.119, 0.259, 2.82, 0.047, 0.143, 0.343, 1.30, 0.432}},
+};
+constexpr double kSmallDtile[2][7] = {{3.09, 0.366, 0, 0.024, 0.045, 2.11, 0.495},
+                                      {3.53, 0.344, 0, 0.036, 0.015, 1.57, 0.451}};
+// The flex tile kernel unsplit at up to 64 rows (terms as in FlexModel).
+constexpr FlexModel kSmallFlex[] = {
+    {222, 64, 64, {1.07, 0.025, 0.224, 0.663, 0.055, 1.69, 0.079}, {}},
+    {224, 64, 128, {3.17, 0.331, 0, 0.619, 0.045, 0, 0.117}, {}},
+};
+
+double flex_us(const double* c, double n, int64_t kbs, double out_mb, double w_mb, double slow) {
+  return c[0] + slow * c[1] * n * kbs + c[2] * kbs + c[3] * out_mb + c[4] * w_mb + c[5] * n +
+         c[6] * std::max(0.0, w_mb - 80.0);
+}
+
+double small_m_us(int width, int S, bool aligned, int nmat, int64_t M, int64_t KB, int64_t NB) {
+  const int mt = M <= 32 ? 1 : 2;
+  const SmallModel* m = nullptr;
+  for (const SmallModel& f : kSmall)
+    if (f.nmat == nmat && f.mt == mt && f.width == width) m = &f;
+  if (!m) return 1e9;
+  const int groups = width == 1 || (nmat == 2 && mt == 1) ? width : width / 2;  // wave groups
+  const int64_t waves = llk_skinny_threads(nmat, (int)M, width) / 64 / groups;
+  const int64_t kbs = (KB + S - 1) / S;
+  const double r = (double)((NB * 4 / width * S + 255) / 256);
+  const double* c = m->c;
+  return c[0] + c[1] * (double)((kbs + waves - 1) / waves) + c[2] * r * kbs * width / 2.0 +
+         c[3] * r + c[4] * KB * NB * 16384e-6 * nmat +
+         c[aligned ? 5 : 6] * r * kbs * groups * M / 32.0 +
+         (S > 1 ? c[7] + c[8] * S * nmat * mt * 32 * NB * 512e-6 : 0.0);
+}
+
+Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, int64_t KB,
+                int64_t NB, const llk_tensor2d* x) {
+  const bool aligned = x_vec_ok(x);
+  const double w_mb = KB * NB * 16384e-6 * nmat;
+  double best;
+  if (ref.dtile) {
+    const int64_t kbs = (KB + ref.S - 1) / ref.S;
+    const double* c = kSmallDtile[nmat - 1];
+    best = c[0] + c[1] * (double)((NB * nmat * ref.S + 255) / 256) * kbs + c[3] * w_mb +
+           c[4] * std::max(0.0, w_mb - 80.0) +
+           (ref.S > 1 ? c[5] + c[6] * ref.S * nmat * ((M + 31) / 32 * 32) * NB * 512e-6 : 0.0);
+  } else {
+    best = small_m_us(ref.G, ref.S, aligned, nmat, M, KB, NB);
+  }
+  // Below these margins the fit's own error chose: 7 of 296 lost 2-10%.
+  best = ref.S > 1 ? 0.96 * (best + 1.0) : 0.86 * best;
+  Plan q;
+  bool taken = false;
+  for (const int width : {1, 2}) {
+    const double us = small_m_us(width, 1, aligned, nmat, M, KB, NB);
+    if (us >= best) continue;
+    best = us;
+    q = Plan{};
+    q.skinny = true;
+    q.G = width;
+    taken = true;
+  }
+  if (KB * NB * nmat <= 8192 && llk_flex_fits(M, K, x->stride0, 0, 0)) {
+    const double y_mb = M * NB * 128 * 3e-6;
+    for (const FlexModel& f : kSmallFlex) {
+      const double n = (double)((NB * 128 * nmat / f.tn + 255) / 256);
+      const double us = flex_us(f.one, n, KB, y_mb, w_mb, 1.0);
+      if (us >= best) continue;
+      best = us;
+      q = Plan{};
+      q.flex = f.cfg;
+      taken = true;
+    }
+  }
+  if (!taken) return p;
+  q.ws_bytes = p.ws_bytes;
+  return q;
+}
+
 // The plan: above 64 rows the flex tile kernel where it is modelled faster.
 // The choice depends on the shape and X's alignment alone -- not on the
 // result type or on the workspace at hand -- so a bf16 result stays the
@@ -831,8 +935,26 @@ double plan_us(const Plan& p, int nmat, int64_t M, int64_t KB, int64_t NB) {
 // record has chosen among those kernels.  A caller's scratch (max_ws) that
 // holds the other plan but not this one's planes gets the other plan.
 Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const llk_tensor2d* x,
-                 size_t max_ws = SIZE_MAX, bool accumulate = false, bool out_bf16 = true) {
+                 size_t max_ws = SIZE_MAX, bool accumulate = false, bool out_bf16 = true,
+                 bool rowmajor = false) {
   Plan p = plan_launch_large(nmat, M, K, KB, NB, x, max_ws, accumulate, out_bf16);
+  p.need = p.ws_bytes;
+  if (M <= 64 && llk::tunable("flex_tile") <= 1) {
+    // The decode tile kernel unsplit, narrower outputs (N <= 2176) and calls for which a knob or a schedule
+    // record has chosen keep their plans, which callers and tests hold this
+    // library to; row-major weights have no small-M form.
+    llk::ScheduleEntry se;
+    if (!x || rowmajor || NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws || llk::tunable("flex_tile") == 0 ||
+        llk::tunable("decode_max_m") != 64 || llk::tunable("decode_splits") > 0 ||
+        llk::tunable("decode_group_width") > 0 || llk::tunable("decode_tile") != 1 ||
+        llk::tunable("decode_target_wgs") != 256 || llk::tunable("decode_min_kb") != 2 ||
+        (db_entry(nmat, M, &se) && (se.grain_size > 0 || se.BN == 32 || se.BN == 64 || se.BN == 128)))
+      return p;
+    const Plan ref = max_ws != SIZE_MAX
+                         ? plan_launch_large(nmat, M, K, KB, NB, x, SIZE_MAX, accumulate, out_bf16)
+                         : p;
+    return small_plan(p, ref, nmat, M, K, KB, NB, x);
+  }
   const int64_t knob = llk::tunable("flex_tile");
   const int64_t forced_s = llk::tunable("tile_splits");
   int cfg = 0;
@@ -876,10 +998,9 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
         if (want > 1 && (tiles * want > 1024 || KB / want < 3)) break;
         const int64_t kbs = (KB + want - 1) / want, s = (KB + kbs - 1) / kbs;
         const double n = (double)((tiles * s + 255) / 256);
-        const double* c = s == 1 ? f.one : f.many;
-        const double us = c[0] + slow * c[1] * n * kbs + c[2] * kbs +
-                          c[3] * (s == 1 ? y_mb : s * nmat * M * NB * 512e-6) + c[4] * w_mb +
-                          c[5] * n + c[6] * std::max(0.0, w_mb - 80.0);
+        const double us =
+            flex_us(s == 1 ? f.one : f.many, n, kbs,
+                    s == 1 ? y_mb : s * nmat * M * NB * 512e-6, w_mb, slow);
         if (us < best) {
           best = us;
           cfg = f.cfg;
@@ -898,7 +1019,7 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
   Plan q;
   q.flex = cfg;
   q.S = (int)S;
-  q.flex_bytes = bytes;
+  q.need = bytes;
   q.ws_bytes = std::max(p.ws_bytes, bytes);
   return q;
 }
@@ -932,19 +1053,21 @@ int run_contraction(int mode, const llk_tensor2d* x, const llk_packed_weights* w
     const Plan q = plan_launch_large(nmat, M, K, w0->KB, w0->NB, x, max_ws, accumulate,
                                      out_dtype == LLK_BF16);
     asked = q.ws_bytes;
-    if (ctx->scratch_size < p.flex_bytes) p = q;
+    if (ctx->scratch_size < p.need) {
+      p = q;
+      p.need = q.ws_bytes;
+    }
   }
   if (p.too_large)
     return fail(LLK_ERR_SHAPE, "%s: K=%lld too large for M=%lld (the tile kernel needs K <= %lld)",
                 what, (long long)K, (long long)M, (long long)(((int64_t)1 << 31) / 512 - 64));
-  if ((p.flex ? p.flex_bytes : p.ws_bytes) > max_ws)
+  if (p.need > max_ws)
     return fail(LLK_ERR_SCRATCH,
                 "%s: M=%lld K=%lld needs %zu workspace bytes, more than the %zu available",
                 what, (long long)M, (long long)K, p.ws_bytes, max_ws);
   void* ws = nullptr;
   Workspace* held = nullptr;
-  int rc = get_workspace(dev, p.flex ? p.flex_bytes : p.ws_bytes, std::min(asked, max_ws), ctx, &ws,
-                         &held);
+  int rc = get_workspace(dev, p.need, std::min(asked, max_ws), ctx, &ws, &held);
   if (rc) return rc;
   hipStream_t s = stream_of(ctx);
   rc = launch_contraction(mode, x, w0, w1, y, out_dtype, p, static_cast<uint8_t*>(ws), s, what,
@@ -1726,7 +1849,8 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   if (wg->stride1 != 1 || (mode == 1 && (!wu || wu->stride1 != 1 || wu->dim1 != N))) return LLK_OK;
   const int nmat = mode == 1 ? 2 : 1;
   const int64_t KB = llk::deviceBlocksK(K), NB = llk::deviceBlocksN(N);
-  const Plan p = plan_launch(nmat, M, K, KB, NB, x, SIZE_MAX, accumulate, out_dtype == LLK_BF16);
+  const Plan p =
+      plan_launch(nmat, M, K, KB, NB, x, SIZE_MAX, accumulate, out_dtype == LLK_BF16, true);
   auto fits = [&](bool (*f)(int, int64_t, int64_t, const void*, int64_t, int64_t)) {
     return f((int)M, K, x->stride0, wg->data, wg->stride0, N) &&
            (mode != 1 || f((int)M, K, x->stride0, wu->data, wu->stride0, N));
@@ -1738,7 +1862,7 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   int64_t head_cols = 0;  // tile form: columns of the unsplit head launch
   if (p.flex) {  // row-major weights of any alignment
     if (!llk_flex_fits(M, K, x->stride0, wg->stride0, mode == 1 ? wu->stride0 : 0)) return LLK_OK;
-    ws_bytes = p.flex_bytes;
+    ws_bytes = p.need;
   } else if (p.dtile && M <= 128) {
     if (!fits(&llk_decode_rowmajor_fits)) return LLK_OK;
   } else if (!p.skinny && mode == 1 && (out_dtype == LLK_BF16 || out_dtype == LLK_FP32) &&
