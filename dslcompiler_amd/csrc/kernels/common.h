@@ -137,38 +137,47 @@ __device__ __forceinline__ uint16_t f32_to_f16_rne(float f) {
   return __builtin_bit_cast(uint16_t, h);
 }
 
+// 4 16-bit elements at any 2-byte aligned address, as 16 bytes above.
+__device__ __forceinline__ uint2 load8_any(const void* p) {
+  uint2 v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 8);
+  return v;
+}
+__device__ __forceinline__ void store8_any(void* p, uint2 v) {
+  __builtin_memcpy(__builtin_assume_aligned(p, 2), &v, 8);
+}
+
 // Stores 4 consecutive n of output row m (OUT: bf16, fp16 or fp32; both
-// 16-bit types rounded to nearest even), bounds-checked.
+// 16-bit types rounded to nearest even), bounds-checked; one store whatever
+// the row's alignment (four for unaligned rows: C += A B, 128 x 640 x 9786,
+// 25.5 us, now 15.9).
 template <int OUT>
 __device__ __forceinline__ void store4(void* y, int64_t ldy, int M, int N, int m, int n,
-                                       const float (&v)[4], bool vec_ok) {
+                                       const float (&v)[4]) {
   if (m >= M || n >= N) return;
-  if (OUT == kOutF16) {
-    uint16_t* dst = reinterpret_cast<uint16_t*>(y) + (size_t)m * ldy + n;
-    if (vec_ok && n + 4 <= N) {
-      u16x4 h = {f32_to_f16_rne(v[0]), f32_to_f16_rne(v[1]), f32_to_f16_rne(v[2]),
-                 f32_to_f16_rne(v[3])};
-      *reinterpret_cast<u16x4*>(dst) = h;
-    } else {
-      for (int r = 0; r < 4; ++r)
-        if (n + r < N) dst[r] = f32_to_f16_rne(v[r]);
-    }
-  } else if (OUT == kOutBF16) {
-    uint16_t* dst = reinterpret_cast<uint16_t*>(y) + (size_t)m * ldy + n;
-    if (vec_ok && n + 4 <= N) {
-      *reinterpret_cast<uint2*>(dst) =
-          make_uint2(f32x2_to_bf16x2_rne(v[0], v[1]), f32x2_to_bf16x2_rne(v[2], v[3]));
-    } else {
-      for (int r = 0; r < 4; ++r)
-        if (n + r < N) dst[r] = f32_to_bf16_rne(v[r]);
-    }
-  } else {
+  if constexpr (OUT == kOutF32) {
     float* dst = reinterpret_cast<float*>(y) + (size_t)m * ldy + n;
-    if (vec_ok && n + 4 <= N) {
-      *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+    if (n + 4 <= N) {
+      store16_any(dst, __builtin_bit_cast(u32x4, f32x4{v[0], v[1], v[2], v[3]}));
     } else {
       for (int r = 0; r < 4; ++r)
         if (n + r < N) dst[r] = v[r];
+    }
+  } else {
+    uint16_t* dst = reinterpret_cast<uint16_t*>(y) + (size_t)m * ldy + n;
+    uint2 h;
+    if constexpr (OUT == kOutF16) {
+      h.x = (uint32_t)f32_to_f16_rne(v[0]) | ((uint32_t)f32_to_f16_rne(v[1]) << 16);
+      h.y = (uint32_t)f32_to_f16_rne(v[2]) | ((uint32_t)f32_to_f16_rne(v[3]) << 16);
+    } else {
+      h = make_uint2(f32x2_to_bf16x2_rne(v[0], v[1]), f32x2_to_bf16x2_rne(v[2], v[3]));
+    }
+    if (n + 4 <= N) {
+      store8_any(dst, h);
+    } else {
+      dst[0] = (uint16_t)h.x;
+      if (n + 1 < N) dst[1] = (uint16_t)(h.x >> 16);
+      if (n + 2 < N) dst[2] = (uint16_t)h.y;
     }
   }
 }
@@ -176,15 +185,15 @@ __device__ __forceinline__ void store4(void* y, int64_t ldy, int M, int N, int m
 // Accumulate mode of the GEMM (C += A B, the micro.mma / linalg.matmul
 // contract): adds the output's existing values at the 4 consecutive n of row
 // m, read in the output type, to v (fp32), before the store rounds it.
-// Bounds and the vector condition as store4.
+// Bounds as store4.
 template <int OUT>
 __device__ __forceinline__ void add_existing4(const void* y, int64_t ldy, int M, int N, int m,
-                                              int n, float (&v)[4], bool vec_ok) {
+                                              int n, float (&v)[4]) {
   if (m >= M || n >= N) return;
-  if (OUT == kOutF32) {
+  if constexpr (OUT == kOutF32) {
     const float* src = reinterpret_cast<const float*>(y) + (size_t)m * ldy + n;
-    if (vec_ok && n + 4 <= N) {
-      const f32x4 c = *reinterpret_cast<const f32x4*>(src);
+    if (n + 4 <= N) {
+      const f32x4 c = __builtin_bit_cast(f32x4, load16_any(src));
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] += c[r];
     } else {
@@ -197,8 +206,8 @@ __device__ __forceinline__ void add_existing4(const void* y, int64_t ldy, int M,
       else return bf16_bits_to_f32(h);
     };
     const uint16_t* src = reinterpret_cast<const uint16_t*>(y) + (size_t)m * ldy + n;
-    if (vec_ok && n + 4 <= N) {
-      const uint2 c = *reinterpret_cast<const uint2*>(src);
+    if (n + 4 <= N) {
+      const uint2 c = load8_any(src);
       v[0] += widen((uint16_t)(c.x & 0xffffu));
       v[1] += widen((uint16_t)(c.x >> 16));
       v[2] += widen((uint16_t)(c.y & 0xffffu));

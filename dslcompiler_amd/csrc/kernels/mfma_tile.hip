@@ -137,7 +137,8 @@ __device__ __forceinline__ void acc_fence(f32x4 (&acc)[8][8]) {
 
 // MODE 0: GEMM (C = X W);  MODE 1: fused SwiGLU.
 // OUT: output element type (kOutBF16, kOutF16 (GEMM only), kOutF32).
-// YVEC: Y rows allow a 4-element vector store (aligned base, ldy % 4 == 0).
+// YVEC: Y rows are 16-byte aligned: non-temporal stores (else cached ones of any
+// alignment, whose shared cache lines L2 joins).
 // SPLIT: store raw fp32 partial accumulators of k split s (see TileArgs).
 // RM: the weights are the caller's row-major matrices (TileArgs::ldw0/1),
 // loaded and read as described at the weight stream below; everything else
@@ -485,9 +486,11 @@ __device__ __forceinline__ void tile_body(TileArgs a) {
   // 128-byte row segments out, 8 rows per instruction, where the accumulator
   // layout would store 8- or 16-byte pieces of 16 rows per instruction
   // (measured: GEMM 4096^3 epilogue 12 -> 3.4 us).  A tile wholly inside Y
-  // (or the partial planes) with 16-byte aligned rows copies 16-byte chunks
-  // unchecked; an edge tile checks each chunk and copies the chunks that
-  // straddle a bound (or unaligned rows) element by element.  The stage ring
+  // (or the partial planes) copies 16-byte chunks unchecked, whatever the rows'
+  // alignment (element stores for unaligned rows: GEMM 1731 x 704 x 4637 35.1
+  // us, now 20.0; SwiGLU 4075 x 576 x 7740 118 -> 76 us, with the wide kernel's
+  // copy-out); an edge tile checks each chunk and copies the chunks that
+  // straddle a bound element by element.  The stage ring
   // is free once every wave is past its last operand read.
   __syncthreads();
   uint8_t* const strip = smem + wave * (128 * kStripRow);
@@ -498,8 +501,8 @@ __device__ __forceinline__ void tile_body(TileArgs a) {
   // (A/B on one box: GEMM 4096^3 fp32 out 97.7 -> 96.2 us, config 3 and
   // the MLP within noise); the k-split planes, which the reduce reads back,
   // keep normal stores.
-  auto strip_out = [&](auto E, auto NT, bool fast, bool al16, uint8_t* gdst, int64_t ld_bytes,
-                       int rows_ok, int cols_ok) {
+  auto strip_out = [&](auto E, auto NT, bool fast, uint8_t* gdst, int64_t ld_bytes, int rows_ok,
+                       int cols_ok) {
     constexpr int kE = decltype(E)::value;
     __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's strip writes are done
     __builtin_amdgcn_wave_barrier();
@@ -510,11 +513,11 @@ __device__ __forceinline__ void tile_body(TileArgs a) {
       const uint4 d = *reinterpret_cast<const uint4*>(strip + row * kStripRow + (lane & 7) * 16);
       uint8_t* const out = gdst + row * ld_bytes + (lane & 7) * 16;
       const int c0 = (lane & 7) * (16 / kE);
-      if (fast || (al16 && row < rows_ok && c0 + 16 / kE <= cols_ok)) {
+      if (fast || (row < rows_ok && c0 + 16 / kE <= cols_ok)) {
         if constexpr (decltype(NT)::value)
           __builtin_nontemporal_store(u32x4{d.x, d.y, d.z, d.w}, reinterpret_cast<u32x4*>(out));
         else
-          *reinterpret_cast<uint4*>(out) = d;
+          store16_any(out, u32x4{d.x, d.y, d.z, d.w});
       } else if (row < rows_ok) {
         const uint32_t w[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
@@ -546,7 +549,7 @@ __device__ __forceinline__ void tile_body(TileArgs a) {
         for (int j = 0; j < 8; ++j)
           *reinterpret_cast<f32x4*>(strip + (j * 16 + mr) * kStripRow + (ii * 16 + h4) * 4) =
               acc[2 * sp + ii][j];
-      strip_out(std::integral_constant<int, 4>{}, std::false_type{}, fast, true,
+      strip_out(std::integral_constant<int, 4>{}, std::false_type{}, fast,
                 reinterpret_cast<uint8_t*>(a.part + ((size_t)split * NMAT + mat) * plane +
                                            (size_t)(m0 + wm * 128) * a.n_pad + col0),
                 (int64_t)a.n_pad * 4, rows_ok, a.n_pad - col0);
@@ -556,8 +559,7 @@ __device__ __forceinline__ void tile_body(TileArgs a) {
   constexpr int NI = (MODE == 1) ? 4 : 8;         // 16-column groups of the wave's output
   constexpr int kElem = (OUT == kOutF32) ? 4 : 2;
   constexpr int kPerStrip = 128 / (16 * kElem);  // 16-column groups per 128-byte strip: 4 or 2
-  const bool al16 = ((reinterpret_cast<uintptr_t>(a.y) | (uintptr_t)(a.ldy * kElem)) & 15) == 0;
-  const bool fast = YVEC && m0 + kTileM <= a.M && n_end <= a.N && al16;
+  const bool fast = m0 + kTileM <= a.M && n_end <= a.N;
   const int n_w = (MODE == 1) ? tn * 128 + wn * 64 : tn * 256 + wn * 128;
   uint8_t* const ybase =
       static_cast<uint8_t*>(a.y) + ((size_t)max(0, m0 + wm * 128) * a.ldy + n_w) * kElem;
@@ -591,8 +593,8 @@ __device__ __forceinline__ void tile_body(TileArgs a) {
         }
       }
     }
-    strip_out(std::integral_constant<int, kElem>{}, std::true_type{}, fast, al16, ybase + sidx * 128,
-              a.ldy * kElem, rows_ok, a.N - (n_w + sidx * 128 / kElem));
+    strip_out(std::integral_constant<int, kElem>{}, std::bool_constant<YVEC>{}, fast,
+              ybase + sidx * 128, a.ldy * kElem, rows_ok, a.N - (n_w + sidx * 128 / kElem));
   }
 }
 
@@ -611,7 +613,7 @@ __global__ __launch_bounds__(kThreads, 1) void mfma_tile_rm_kernel(TileArgs a) {
 // Sums the S partial planes of each output element in split order (fixed,
 // so results are reproducible) and applies the epilogue.  One thread per
 // 4 consecutive n of a row.
-template <int MODE, int OUT, bool YVEC>
+template <int MODE, int OUT>
 __global__ __launch_bounds__(256) void split_reduce_kernel(TileArgs a) {
   constexpr int NMAT = (MODE == 1) ? 2 : 1;
   const int quads = (a.N + 3) / 4;
@@ -637,9 +639,9 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(TileArgs a) {
       v[q] = sum[0][q];
   }
   if constexpr (MODE == 0) {
-    if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, YVEC);
+    if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
   }
-  store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, YVEC);
+  store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
 }
 
 // ---------------------------------------------------------------------------
@@ -656,19 +658,19 @@ const char* tile_symbol() {
   return name.c_str();
 }
 
-template <int MODE, int OUT, bool YVEC>
+template <int MODE, int OUT>
 const char* split_reduce_symbol() {
   static const std::string name = "_ZN10llk_gfx95019split_reduce_kernelI" + mangle_int(MODE) +
-                                  mangle_int(OUT) + mangle_bool(YVEC) + "EEvNS_8TileArgsE";
+                                  mangle_int(OUT) + "EEvNS_8TileArgsE";
   return name.c_str();
 }
 
 // The reduce of a k split's planes into y.
-template <int MODE, int OUT, bool YVEC>
+template <int MODE, int OUT>
 static hipError_t launch_reduce(const TileArgs& a, const llk::ModuleFns* mod, hipStream_t s) {
   const int64_t threads = (int64_t)a.M * ((a.N + 3) / 4);
-  return launch_kernel(mod, reinterpret_cast<const void*>(split_reduce_kernel<MODE, OUT, YVEC>),
-                       &split_reduce_symbol<MODE, OUT, YVEC>,
+  return launch_kernel(mod, reinterpret_cast<const void*>(split_reduce_kernel<MODE, OUT>),
+                       &split_reduce_symbol<MODE, OUT>,
                        dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a);
 }
 
@@ -692,18 +694,18 @@ static hipError_t launch_tile_t(const TileArgs& a, const llk::ModuleFns* mod, hi
 
 // A k-split (or accumulating) launch: the tile kernel's fp32 partial planes,
 // then split_reduce_kernel.
-template <int MODE, int OUT, bool YVEC, bool RM = false>
+template <int MODE, int OUT, bool RM = false>
 static hipError_t launch_split(const TileArgs& a, const llk::ModuleFns* mod, hipStream_t s) {
   // Partials are fp32 planes with 16-byte aligned rows: one instantiation.
   hipError_t e = launch_tile_t<MODE, kOutF32, true, true, RM>(a, mod, s);
   if (e != hipSuccess) return e;
-  return launch_reduce<MODE, OUT, YVEC>(a, mod, s);
+  return launch_reduce<MODE, OUT>(a, mod, s);
 }
 
 template <int MODE, int OUT, bool YVEC, bool RM = false>
 static hipError_t launch_t(const TileArgs& a, const llk::ModuleFns* mod, hipStream_t s) {
   if (a.S <= 1 && !a.accumulate) return launch_tile_t<MODE, OUT, YVEC, false, RM>(a, mod, s);
-  return launch_split<MODE, OUT, YVEC, RM>(a, mod, s);
+  return launch_split<MODE, OUT, RM>(a, mod, s);
 }
 
 template <int MODE, int OUT>
@@ -787,7 +789,7 @@ hipError_t llk_launch_tile(int mode, const uint16_t* x, int64_t ldx, const void*
 // k split left, in split order, applies the epilogue of `mode` (1 SwiGLU, 0
 // GEMM, with accumulate y += sum) and stores y.
 hipError_t llk_launch_split_reduce(int mode, const void* part, int S, void* y, int64_t ldy, int M,
-                                   int N, int NB, int out, bool yvec, bool accumulate,
+                                   int N, int NB, int out, bool accumulate,
                                    const llk::ModuleFns* mod, hipStream_t s) {
   using namespace llk_gfx950;
   if (part == nullptr || S < 1 || M < 1 || N < 1 || (accumulate && mode != 0))
@@ -802,23 +804,13 @@ hipError_t llk_launch_split_reduce(int mode, const void* part, int S, void* y, i
   a.part = static_cast<float*>(const_cast<void*>(part));
   a.accumulate = accumulate ? 1 : 0;
 #if !defined(LLK_CO_OP) || LLK_CO_OP == 1
-  if (mode == 1 && out == kOutBF16)
-    return yvec ? launch_reduce<1, kOutBF16, true>(a, mod, s)
-                : launch_reduce<1, kOutBF16, false>(a, mod, s);
-  if (mode == 1 && out == kOutF32)
-    return yvec ? launch_reduce<1, kOutF32, true>(a, mod, s)
-                : launch_reduce<1, kOutF32, false>(a, mod, s);
+  if (mode == 1 && out == kOutBF16) return launch_reduce<1, kOutBF16>(a, mod, s);
+  if (mode == 1 && out == kOutF32) return launch_reduce<1, kOutF32>(a, mod, s);
 #endif
 #if !defined(LLK_CO_OP) || LLK_CO_OP == 0
-  if (mode == 0 && out == kOutBF16)
-    return yvec ? launch_reduce<0, kOutBF16, true>(a, mod, s)
-                : launch_reduce<0, kOutBF16, false>(a, mod, s);
-  if (mode == 0 && out == kOutF16)
-    return yvec ? launch_reduce<0, kOutF16, true>(a, mod, s)
-                : launch_reduce<0, kOutF16, false>(a, mod, s);
-  if (mode == 0 && out == kOutF32)
-    return yvec ? launch_reduce<0, kOutF32, true>(a, mod, s)
-                : launch_reduce<0, kOutF32, false>(a, mod, s);
+  if (mode == 0 && out == kOutBF16) return launch_reduce<0, kOutBF16>(a, mod, s);
+  if (mode == 0 && out == kOutF16) return launch_reduce<0, kOutF16>(a, mod, s);
+  if (mode == 0 && out == kOutF32) return launch_reduce<0, kOutF32>(a, mod, s);
 #endif
   return hipErrorInvalidValue;
 }
@@ -885,15 +877,9 @@ hipError_t llk_launch_tile_rowmajor(int mode, const uint16_t* x, int64_t ldx, co
 #endif
 #if !defined(LLK_CO_OP) || LLK_CO_OP == 0
   if (mode == 0) {  // accumulating: the planes and the reduce, which reads y
-    if (out == kOutBF16)
-      return yvec ? launch_split<0, kOutBF16, true, true>(a, mod, s)
-                  : launch_split<0, kOutBF16, false, true>(a, mod, s);
-    if (out == kOutF16)
-      return yvec ? launch_split<0, kOutF16, true, true>(a, mod, s)
-                  : launch_split<0, kOutF16, false, true>(a, mod, s);
-    if (out == kOutF32)
-      return yvec ? launch_split<0, kOutF32, true, true>(a, mod, s)
-                  : launch_split<0, kOutF32, false, true>(a, mod, s);
+    if (out == kOutBF16) return launch_split<0, kOutBF16, true>(a, mod, s);
+    if (out == kOutF16) return launch_split<0, kOutF16, true>(a, mod, s);
+    if (out == kOutF32) return launch_split<0, kOutF32, true>(a, mod, s);
   }
 #endif
   return hipErrorInvalidValue;

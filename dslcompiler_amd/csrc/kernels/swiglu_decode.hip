@@ -33,7 +33,6 @@ struct SkinnyArgs {
   float* part;        // [S][NMAT][MT*32][n_pad] fp32 partials (S > 1)
   int64_t ldx, ldy;
   int M, N, K, KB, NB, S, kb_per_split, n_pad;
-  bool yvec;
   bool accumulate;  // GEMM only: y += x w (the existing y read in its type)
 };
 
@@ -267,9 +266,9 @@ __global__ __launch_bounds__(KS * G * 64) void skinny_kernel(SkinnyArgs a) {
           v[q] = sum[i][0][q];
       }
       if constexpr (NMAT == 1) {
-        if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, a.yvec);
+        if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
       }
-      store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, a.yvec);
+      store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
     }
   }
 }
@@ -299,9 +298,9 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(SkinnyArgs a, int ro
       v[q] = s[0][q];
   }
   if constexpr (NMAT == 1) {
-    if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, a.yvec);
+    if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
   }
-  store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, a.yvec);
+  store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
 }
 
 // Launch shape for (NMAT, MT) and a workgroup width of W 32-column groups:
@@ -467,7 +466,6 @@ struct DecTileArgs {
   float* part;        // [S][NMAT][rows][n_pad] fp32 partials (S > 1)
   int64_t ldx, ldy;
   int M, N, KB, NB, S, kbs, n_pad, rows;
-  bool yvec;
   bool accumulate;  // GEMM only, S == 1: y += x w (the existing y read in its type)
   // The row-major form (RM): w0 / w1 are bf16 [K, N] with rows of ldw0 /
   // ldw1 elements instead of packed payloads.
@@ -717,7 +715,7 @@ __global__ __launch_bounds__(256) void decode_tile_kernel(DecTileArgs a) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           v[q] = swiglu_act(acc[0][t][4 * g + q], acc[1][t][4 * g + q]);
-        store4<OUT>(a.y, a.ldy, a.M, a.N, m, n_col + n_off, v, a.yvec);
+        store4<OUT>(a.y, a.ldy, a.M, a.N, m, n_col + n_off, v);
       } else {
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
@@ -725,8 +723,8 @@ __global__ __launch_bounds__(256) void decode_tile_kernel(DecTileArgs a) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) v[q] = acc[p][t][4 * g + q];
           const int n = n_col + p * 64 + n_off;
-          if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, a.yvec);
-          store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v, a.yvec);
+          if (a.accumulate) add_existing4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
+          store4<OUT>(a.y, a.ldy, a.M, a.N, m, n, v);
         }
       }
     }
@@ -764,7 +762,6 @@ static hipError_t launch_decode_tile_t(const DecTileArgs& a, const llk::ModuleFn
   r.N = a.N;
   r.S = a.S;
   r.n_pad = a.n_pad;
-  r.yvec = a.yvec;
   r.accumulate = a.accumulate;
   const int64_t threads = (int64_t)a.M * (a.n_pad / 4);
   return launch_kernel(mod, reinterpret_cast<const void*>(skinny_reduce_kernel<NMAT, OUT>),
@@ -814,7 +811,7 @@ size_t llk_skinny_workspace_bytes(int nmat, int M, int N_pad, int S) {
 // 128*NB, S) bytes when S > 1.
 hipError_t llk_launch_skinny(int mode, const uint16_t* x, int64_t ldx, const void* w0,
                              const void* w1, void* y, int64_t ldy, int M, int N, int K, int KB,
-                             int NB, int S, int G, void* ws, int out, bool xvec, bool yvec,
+                             int NB, int S, int G, void* ws, int out, bool xvec,
                              bool accumulate, const llk::ModuleFns* mod, hipStream_t s) {
   using namespace llk_gfx950;
   if (M < 1 || M > 64 || (G != 1 && G != 2 && G != 4)) return hipErrorInvalidValue;
@@ -833,7 +830,6 @@ hipError_t llk_launch_skinny(int mode, const uint16_t* x, int64_t ldx, const voi
   a.S = S < 1 ? 1 : S;
   a.kb_per_split = (KB + a.S - 1) / a.S;
   a.n_pad = NB * kPackN;
-  a.yvec = yvec;
   a.accumulate = accumulate;
   a.part = static_cast<float*>(ws);
   if (accumulate && mode != 0) return hipErrorInvalidValue;
@@ -884,7 +880,7 @@ bool llk_decode_rowmajor_fits(int M, int64_t K, int64_t ldx, const void* w, int6
 // only) adds the existing y.
 hipError_t llk_launch_decode_tile(int mode, const uint16_t* x, int64_t ldx, const void* w0,
                                   const void* w1, void* y, int64_t ldy, int M, int N, int KB,
-                                  int NB, int S, void* ws, int out, bool yvec, bool accumulate,
+                                  int NB, int S, void* ws, int out, bool accumulate,
                                   const llk::ModuleFns* mod, hipStream_t s) {
   using namespace llk_gfx950;
   if (!llk_decode_tile_fits(M, (int64_t)KB * 64, ldx) || NB < 1 || (accumulate && mode != 0))
@@ -905,7 +901,6 @@ hipError_t llk_launch_decode_tile(int mode, const uint16_t* x, int64_t ldx, cons
   a.kbs = (KB + a.S - 1) / a.S;
   a.n_pad = NB * kPackN;
   a.rows = skinny_rows(M);
-  a.yvec = yvec;
   a.accumulate = accumulate;
   if (a.S > 1 && (ws == nullptr || (int64_t)(a.S - 1) * a.kbs >= KB)) return hipErrorInvalidValue;
   const int mt = dec_mt(M);
@@ -933,7 +928,7 @@ hipError_t llk_launch_decode_tile(int mode, const uint16_t* x, int64_t ldx, cons
 hipError_t llk_launch_decode_rowmajor(int mode, const uint16_t* x, int64_t ldx,
                                       const uint16_t* w0, int64_t ldw0, const uint16_t* w1,
                                       int64_t ldw1, void* y, int64_t ldy, int M, int N, int K,
-                                      int S, void* ws, int out, bool yvec, bool accumulate,
+                                      int S, void* ws, int out, bool accumulate,
                                       const llk::ModuleFns* mod, hipStream_t s) {
   using namespace llk_gfx950;
   if (N < 1 || !llk_decode_rowmajor_fits(M, K, ldx, w0, ldw0, N) ||
@@ -958,7 +953,6 @@ hipError_t llk_launch_decode_rowmajor(int mode, const uint16_t* x, int64_t ldx,
   a.kbs = (a.KB + a.S - 1) / a.S;
   a.n_pad = a.NB * kPackN;
   a.rows = skinny_rows(M);
-  a.yvec = yvec;
   a.accumulate = accumulate;
   if (a.S > 1 && (ws == nullptr || (int64_t)(a.S - 1) * a.kbs >= a.KB)) return hipErrorInvalidValue;
   const int mt = dec_mt(M);

@@ -509,6 +509,9 @@ __global__ __launch_bounds__(256, 1) void mfma_swiglu_wide_kernel(WideArgs a) {
     uint16_t* const out = a.y + (size_t)m * a.ldy + n;
     if (fast || (al16 && n + 8 <= a.N)) {
       __builtin_nontemporal_store(u32x4{d.x, d.y, d.z, d.w}, reinterpret_cast<u32x4*>(out));
+    } else if (n + 8 <= a.N) {
+      // Unaligned rows: chunks share cache lines, which L2 joins.
+      store16_any(out, u32x4{d.x, d.y, d.z, d.w});
     } else {
       const uint32_t w[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
@@ -555,8 +558,7 @@ __global__ __launch_bounds__(256) void wide_reduce_kernel(WideArgs a) {
   float v[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) v[q] = swiglu_act(g[q], u[q]);
-  const bool vec = ((reinterpret_cast<uintptr_t>(a.y) | (uintptr_t)(a.ldy * 2)) & 7) == 0;
-  store4<kOutBF16>(a.y, a.ldy, a.M, a.N, m, n, v, vec);
+  store4<kOutBF16>(a.y, a.ldy, a.M, a.N, m, n, v);
 }
 
 template <int B, bool SPLIT, bool WNT>

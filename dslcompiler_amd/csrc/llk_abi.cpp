@@ -46,21 +46,21 @@ size_t llk_swiglu_wide_split_bytes(int B, int M, int N, int S);
 hipError_t llk_launch_skinny(int mode, const uint16_t* x, int64_t ldx, const void* w0,
                              const void* w1, void* y, int64_t ldy, int M, int N, int K, int KB,
                              int NB, int S, int G, void* ws, int out_dtype, bool xvec,
-                             bool yvec, bool accumulate, const llk::ModuleFns* mod,
+                             bool accumulate, const llk::ModuleFns* mod,
                              hipStream_t s);
 size_t llk_skinny_workspace_bytes(int nmat, int M, int N_pad, int S);
 int llk_skinny_threads(int nmat, int M, int G);
 bool llk_decode_tile_fits(int M, int64_t K, int64_t ldx);
 hipError_t llk_launch_decode_tile(int mode, const uint16_t* x, int64_t ldx, const void* w0,
                                   const void* w1, void* y, int64_t ldy, int M, int N, int KB,
-                                  int NB, int S, void* ws, int out, bool yvec, bool accumulate,
+                                  int NB, int S, void* ws, int out, bool accumulate,
                                   const llk::ModuleFns* mod, hipStream_t s);
 bool llk_decode_rowmajor_fits(int M, int64_t K, int64_t ldx, const void* w, int64_t ldw,
                               int64_t N);
 hipError_t llk_launch_decode_rowmajor(int mode, const uint16_t* x, int64_t ldx,
                                       const uint16_t* w0, int64_t ldw0, const uint16_t* w1,
                                       int64_t ldw1, void* y, int64_t ldy, int M, int N, int K,
-                                      int S, void* ws, int out, bool yvec, bool accumulate,
+                                      int S, void* ws, int out, bool accumulate,
                                       const llk::ModuleFns* mod, hipStream_t s);
 bool llk_tile_rowmajor_fits(int M, int64_t K, int64_t ldx, const void* w, int64_t ldw, int64_t N);
 hipError_t llk_launch_tile_rowmajor(int mode, const uint16_t* x, int64_t ldx, const uint16_t* w0,
@@ -74,7 +74,7 @@ hipError_t llk_launch_flex(int mode, int cfg, const uint16_t* x, int64_t ldx, co
                            int M, int N, int K, int S, void* part, int out, bool accumulate,
                            bool rowmajor, const llk::ModuleFns* mod, hipStream_t s);
 hipError_t llk_launch_split_reduce(int mode, const void* part, int S, void* y, int64_t ldy, int M,
-                                   int N, int NB, int out, bool yvec, bool accumulate,
+                                   int N, int NB, int out, bool accumulate,
                                    const llk::ModuleFns* mod, hipStream_t s);
 hipError_t llk_launch_pad_rows(const uint16_t* x, int64_t ldx, int M, int K, uint16_t* out,
                                int64_t ldo, const llk::ModuleFns* mod, hipStream_t s);
@@ -186,10 +186,9 @@ bool x_vec_ok(const llk_tensor2d* x) {
          (x->dim1 % 8 == 0);
 }
 size_t dtype_size(int dtype) { return dtype == LLK_FP32 ? 4 : 2; }
-// Rows allow a 4-element vector store.
+// Rows are 16-byte aligned.
 bool y_vec_ok(const llk_tensor2d* y, int dtype) {
-  const uintptr_t align = 4 * dtype_size(dtype);
-  return (reinterpret_cast<uintptr_t>(y->data) % align == 0) && (y->stride0 % 4 == 0);
+  return reinterpret_cast<uintptr_t>(y->data) % 16 == 0 && y->stride0 * dtype_size(dtype) % 16 == 0;
 }
 
 // Key of the library workspace of a stream: the stream handle, and for the
@@ -1090,14 +1089,14 @@ int launch_contraction(int mode, const llk_tensor2d* x, const llk_packed_weights
                         body, out_dtype, accumulate, false, mod, s);
     if (e == hipSuccess && p.S > 1)
       e = llk_launch_split_reduce(mode, body, p.S, y->data, y->stride0, (int)M, (int)N, (int)w0->NB,
-                                  out_dtype, yvec, accumulate, mod, s);
+                                  out_dtype, accumulate, mod, s);
     if (e != hipSuccess) return fail_hip(e, what);
     return LLK_OK;
   }
   if (p.dtile) {
     e = llk_launch_decode_tile(mode, static_cast<const uint16_t*>(x->data), x->stride0, w0->dev,
                                w1 ? w1->dev : nullptr, y->data, y->stride0, (int)M, (int)N,
-                               (int)w0->KB, (int)w0->NB, p.S, body, out_dtype, yvec, accumulate,
+                               (int)w0->KB, (int)w0->NB, p.S, body, out_dtype, accumulate,
                                mod, s);
     if (e != hipSuccess) return fail_hip(e, what);
     return LLK_OK;
@@ -1105,7 +1104,7 @@ int launch_contraction(int mode, const llk_tensor2d* x, const llk_packed_weights
   if (p.skinny) {
     e = llk_launch_skinny(mode, static_cast<const uint16_t*>(x->data), x->stride0, w0->dev,
                           w1 ? w1->dev : nullptr, y->data, y->stride0, (int)M, (int)N, (int)K,
-                          (int)w0->KB, (int)w0->NB, p.S, p.G, body, out_dtype, x_vec_ok(x), yvec,
+                          (int)w0->KB, (int)w0->NB, p.S, p.G, body, out_dtype, x_vec_ok(x),
                           accumulate, mod, s);
     if (e != hipSuccess) return fail_hip(e, what);
     return LLK_OK;
@@ -1900,7 +1899,7 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
                         ws, out_dtype, accumulate, true, mod, s);
     if (e == hipSuccess && S > 1)
       e = llk_launch_split_reduce(mode, ws, S, y->data, y->stride0, (int)M, (int)N, (int)NB,
-                                  out_dtype, y_vec_ok(y, out_dtype), accumulate, mod, s);
+                                  out_dtype, accumulate, mod, s);
   } else if (tile) {
     // head columns unsplit, then the rest with the plan's splits (offsets of
     // 128-column multiples keep every row 16-byte aligned)
@@ -1919,7 +1918,7 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   } else {
     e = llk_launch_decode_rowmajor(mode, xd, x->stride0, wgd, wg->stride0, wud,
                                    mode == 1 ? wu->stride0 : 0, y->data, y->stride0, (int)M, (int)N,
-                                   (int)K, S, ws, out_dtype, y_vec_ok(y, out_dtype), accumulate,
+                                   (int)K, S, ws, out_dtype, accumulate,
                                    mod, s);
   }
   release_workspace(dev, held, s);
