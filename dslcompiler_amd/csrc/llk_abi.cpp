@@ -1860,7 +1860,12 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   bool tile = false;
   int64_t head_cols = 0;  // tile form: columns of the unsplit head launch
   if (p.flex) {  // row-major weights of any alignment
-    if (!llk_flex_fits(M, K, x->stride0, wg->stride0, mode == 1 ? wu->stride0 : 0)) return LLK_OK;
+    // A row's last 16-byte chunk ends up to 7 elements past column N, in the
+    // next row (the last row is read by the element): rows at least 8 apart.
+    const int64_t ldw = mode == 1 ? std::min(wg->stride0, wu->stride0) : wg->stride0;
+    if (ldw < std::max<int64_t>(N, 8) ||
+        !llk_flex_fits(M, K, x->stride0, wg->stride0, mode == 1 ? wu->stride0 : 0))
+      return LLK_OK;
     ws_bytes = p.need;
   } else if (p.dtile && M <= 128) {
     if (!fits(&llk_decode_rowmajor_fits)) return LLK_OK;

@@ -99,7 +99,8 @@ def test_flex_accumulates_into_a_view(llk, gpu, cfg, N, shift):
 
 @pytest.mark.parametrize("cfg", TILES)
 @pytest.mark.parametrize("M,N,K,ldw,S", [(65, 129, 72, 131, 1), (130, 40, 640, 40, 1),
-                                        (70, 1, 64, 1, 1), (129, 300, 1000, 301, 3)])
+                                        (70, 1, 64, 1, 1), (70, 1, 640, 1, 1), (70, 3, 200, 8, 1),
+                                        (129, 300, 1000, 301, 3)])
 def test_flex_row_major_weights(llk, gpu, cfg, M, N, K, ldw, S):
     """The KernelFn on device weights of any stride and alignment: the packed
     path's bits; rows of Inf past the last column change nothing."""
