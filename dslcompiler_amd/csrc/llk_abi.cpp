@@ -939,12 +939,13 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
   Plan p = plan_launch_large(nmat, M, K, KB, NB, x, max_ws, accumulate, out_bf16);
   p.need = p.ws_bytes;
   if (M <= 64 && llk::tunable("flex_tile") <= 1) {
-    // The decode tile kernel unsplit, narrower outputs (N <= 2176) and calls for which a knob or a schedule
-    // record has chosen keep their plans, which callers and tests hold this
-    // library to; row-major weights have no small-M form.
+    // The decode tile kernel unsplit, narrower outputs (N <= 2176) and calls for
+    // which a knob or a schedule record has chosen keep their plans, which
+    // callers and tests hold this library to; row-major weights have no small-M
+    // form.
     llk::ScheduleEntry se;
-    if (!x || rowmajor || NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws || llk::tunable("flex_tile") == 0 ||
-        llk::tunable("decode_max_m") != 64 || llk::tunable("decode_splits") > 0 ||
+    if (!x || rowmajor || NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws ||
+        llk::tunable("flex_tile") == 0 || llk::tunable("decode_max_m") != 64 || llk::tunable("decode_splits") > 0 ||
         llk::tunable("decode_group_width") > 0 || llk::tunable("decode_tile") != 1 ||
         llk::tunable("decode_target_wgs") != 256 || llk::tunable("decode_min_kb") != 2 ||
         (db_entry(nmat, M, &se) && (se.grain_size > 0 || se.BN == 32 || se.BN == 64 || se.BN == 128)))
@@ -964,8 +965,8 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     S = (KB + kbs - 1) / kbs;
   } else {
     if (knob == 0 || M <= 64 || KB <= (accumulate ? 12 : 8) ||
-        KB * NB * nmat > 8192 || (p.chunk > 0 && p.chunk < M) || p.too_large || p.ws_bytes > max_ws || forced_s > 0 ||
-        llk::tunable("tile_wide") != 1 || llk::tunable("tile_wgs_per_wave") != 256 ||
+        KB * NB * nmat > 8192 || (p.chunk > 0 && p.chunk < M) || p.too_large ||
+        p.ws_bytes > max_ws || forced_s > 0 || llk::tunable("tile_wide") != 1 || llk::tunable("tile_wgs_per_wave") != 256 ||
         llk::tunable("tile_tail_split") != 1 || llk::tunable("tile_min_kb") != 4 ||
         llk::tunable("midm_max_m") != 128 || llk::tunable("decode_tile") != 1 ||
         llk::tunable("decode_splits") > 0)
