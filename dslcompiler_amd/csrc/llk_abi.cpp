@@ -766,7 +766,8 @@ Plan plan_launch_large(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
 // 370 random shapes (M 65..4097, K 512..13824, N 512..14336, both operations;
 // each model within 4-10% rms, the tile kernel's unsplit one 15%).  Over them
 // the choice the models make runs 1.42x the plan without this kernel in the
-// geometric mean; always taking the fastest measured would give 1.43x.
+// geometric mean, always taking the fastest measured 1.43x, both before the
+// limit of chain_steps on the sums' length.
 //   us = a + b n kbs + c kbs + d (MB of Y, or of planes when S > 1)
 //          + e (MB of weights) + f n + g (MB of weights beyond 80)
 // with n = ceil(workgroups / 256) and kbs = 64-k steps per split: the
@@ -831,7 +832,7 @@ double plan_us(const Plan& p, int nmat, int64_t M, int64_t KB, int64_t NB) {
 // the host too: 1 us.  Over the 296 shapes with N > 2176 the choice is 1.11x
 // the plan without it in the geometric mean of device time; M x N x K: GEMM
 // 2 x 2648 x 640 6.8 -> 3.9 us, 56 x 8560 x 4035 41.4 -> 23.7 us, SwiGLU
-// 60 x 5389 x 961 19.3 -> 9.3 us, 2 x 7163 x 1920 13.2 -> 11.4 us; none lost.
+// 2 x 7163 x 1920 13.2 -> 11.4 us; none lost (before the limit of chain_steps).
 struct SmallModel {
   int nmat, mt, width;
   double c[9];
@@ -859,6 +860,24 @@ double flex_us(const double* c, double n, int64_t kbs, double out_mb, double w_m
          c[6] * std::max(0.0, w_mb - 80.0);
 }
 
+// Small-M kernel: waves of a workgroup that share a column group's k.
+int small_m_k_waves(int nmat, int64_t M, int width) {
+  const int groups = width == 1 || (nmat == 2 && M <= 32) ? width : width / 2;  // wave groups
+  return llk_skinny_threads(nmat, (int)M, width) / 64 / groups;
+}
+
+// 64-k steps that a plan sums in one accumulator.  The rounding error of an
+// fp32 result grows with their number's root (GEMM 191 x 2112 x 3312: 1.1e-7
+// in seven splits, 2.8e-7 in one; SwiGLU 151 x 3008 x 1392 1.9e-7 in eight,
+// 5.2e-7).  A plan gives way only to one whose sums are no longer, whatever the
+// result type: a bf16 result is the rounding of the fp32 one.
+int64_t chain_steps(const Plan& p, int nmat, int64_t M, int64_t KB) {
+  const int64_t kbs = (KB + p.S - 1) / p.S;
+  if (!p.skinny || p.dtile) return kbs;
+  const int waves = std::max(1, small_m_k_waves(nmat, M, p.G));
+  return (kbs + waves - 1) / waves;
+}
+
 double small_m_us(int width, int S, bool aligned, int nmat, int64_t M, int64_t KB, int64_t NB) {
   const int mt = M <= 32 ? 1 : 2;
   const SmallModel* m = nullptr;
@@ -866,7 +885,7 @@ double small_m_us(int width, int S, bool aligned, int nmat, int64_t M, int64_t K
     if (f.nmat == nmat && f.mt == mt && f.width == width) m = &f;
   if (!m) return 1e9;
   const int groups = width == 1 || (nmat == 2 && mt == 1) ? width : width / 2;  // wave groups
-  const int64_t waves = llk_skinny_threads(nmat, (int)M, width) / 64 / groups;
+  const int64_t waves = small_m_k_waves(nmat, M, width);
   const int64_t kbs = (KB + S - 1) / S;
   const double r = (double)((NB * 4 / width * S + 255) / 256);
   const double* c = m->c;
@@ -879,6 +898,7 @@ double small_m_us(int width, int S, bool aligned, int nmat, int64_t M, int64_t K
 Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, int64_t KB,
                 int64_t NB, const llk_tensor2d* x) {
   const bool aligned = x_vec_ok(x);
+  const int64_t longest = chain_steps(ref, nmat, M, KB);
   const double w_mb = KB * NB * 16384e-6 * nmat;
   double best;
   if (ref.dtile) {
@@ -897,13 +917,15 @@ Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, 
   for (const int width : {1, 2}) {
     const double us = small_m_us(width, 1, aligned, nmat, M, KB, NB);
     if (us >= best) continue;
+    Plan w;
+    w.skinny = true;
+    w.G = width;
+    if (chain_steps(w, nmat, M, KB) > longest) continue;
     best = us;
-    q = Plan{};
-    q.skinny = true;
-    q.G = width;
+    q = w;
     taken = true;
   }
-  if (KB * NB * nmat <= 8192 && llk_flex_fits(M, K, x->stride0, 0, 0)) {
+  if (KB <= longest && KB * NB * nmat <= 8192 && llk_flex_fits(M, K, x->stride0, 0, 0)) {
     const double y_mb = M * NB * 128 * 3e-6;
     for (const FlexModel& f : kSmallFlex) {
       const double n = (double)((NB * 128 * nmat / f.tn + 255) / 256);
@@ -973,9 +995,15 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
       return p;
     llk::ScheduleEntry se;
     if (db_entry(nmat, M, &se) && se.grain_size > 0) return p;
-    const Plan ref = accumulate || !out_bf16 || max_ws != SIZE_MAX
+    const bool any = accumulate || max_ws != SIZE_MAX;
+    const Plan ref = any || !out_bf16
                          ? plan_launch_large(nmat, M, K, KB, NB, x, SIZE_MAX, false, true)
                          : p;
+    Plan ref32 = nmat == 1 ? ref : p;
+    if (nmat == 2 && (any || out_bf16))
+      ref32 = plan_launch_large(nmat, M, K, KB, NB, x, SIZE_MAX, false, false);
+    const int64_t longest =
+        std::min(chain_steps(ref, nmat, M, KB), chain_steps(ref32, nmat, M, KB));
     // X rows that start inside a 128-byte line (whose lines are read twice)
     // slow a step by 8%, rows off the 16 bytes by 20% and at odd elements by
     // 25% (K = 1600 against 1599 and 1598, N = 4288, M = 3779: 60.8, 67.1 and
@@ -997,6 +1025,7 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
       for (const int64_t want : {1, 2, 3, 4, 6, 8, 12, 16}) {
         if (want > 1 && (tiles * want > 1024 || KB / want < 3)) break;
         const int64_t kbs = (KB + want - 1) / want, s = (KB + kbs - 1) / kbs;
+        if (kbs > longest) continue;
         const double n = (double)((tiles * s + 255) / 256);
         const double us =
             flex_us(s == 1 ? f.one : f.many, n, kbs,

@@ -16,13 +16,13 @@ pytestmark = pytest.mark.gpu
 # (op, M, N, K, X aligned, the kernel chosen, its k splits)
 CASES = [
     ("matmul", 7, 2560, 1280, True, "small_m", 1),
-    ("matmul", 64, 2177, 65, False, "flex_tile", 1),      # the first width of the rule
+    ("matmul", 64, 2177, 65, False, "small_m", 1),        # the first width of the rule
     ("matmul", 32, 2176, 520, True, "small_m", 1),        # ... and the last one below it
     ("matmul", 40, 2880, 768, True, "small_m", 1),
     ("fused_swiglu", 1, 2305, 520, True, "small_m", 1),
     ("fused_swiglu", 64, 2944, 576, True, "decode_tile", 1),
-    ("fused_swiglu", 33, 4097, 1031, False, "flex_tile", 1),
-    ("fused_swiglu", 41, 8496, 2241, False, "flex_tile", 1),
+    ("fused_swiglu", 33, 4097, 1031, False, "small_m", 1),
+    ("fused_swiglu", 41, 8496, 2241, False, "small_m", 1),
 ]
 
 

@@ -1,0 +1,38 @@
+"""Results wider than bf16: the plan the dispatcher takes sums no more k in one
+accumulator than the plan without the flex tile kernel and the one-launch
+rule, whose fp32 results it must not be further off than."""
+from __future__ import annotations
+
+import random
+
+import pytest
+
+import dslcompiler_amd as llk
+
+
+def _longest(plan, op, M, K):
+    """64-k steps in one accumulator (the small-M kernel's waves share k)."""
+    steps = -(-((K + 63) // 64) // plan["splits"])
+    if plan["kernel"] != "small_m":
+        return steps
+    width = plan["group_width"]
+    groups = width if width == 1 or (op == "fused_swiglu" and M <= 32) else width // 2
+    return -(-steps // (plan["threads_per_workgroup"] // 64 // groups))
+
+
+@pytest.mark.parametrize("op", ["fused_swiglu", "matmul"])
+@pytest.mark.parametrize("rows", [(1, 64), (65, 1000)])
+def test_sums_no_longer(op, rows):
+    rng = random.Random(rows[1])
+    for _ in range(150):
+        M, K, N = rng.randint(*rows), rng.randint(512, 6000), rng.randint(1376, 14336)
+        if rng.random() < 0.6:
+            K -= K % 64
+        kw = dict(x_aligned=K % 8 == 0, out_f32=True)
+        new = llk.describe_launch(op, M, N, K, **kw)
+        llk.set_tunable("flex_tile", 0)
+        try:
+            old = llk.describe_launch(op, M, N, K, **kw)
+        finally:
+            llk.set_tunable("flex_tile", 1)
+        assert _longest(new, op, M, K) <= _longest(old, op, M, K), (op, M, K, N, new, old)
