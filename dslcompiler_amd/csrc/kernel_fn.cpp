@@ -6,8 +6,8 @@
 // (swiglu_vector_avx2.cpp:278-285 passes the caller's buffers straight
 // through), so by default so does this one.  Device-resident weights with
 // 16-byte aligned rows go straight to a row-major form of the kernels --
-// the decode tile kernel's at most 128 rows of X (the same launch and bits
-// as the packed path), the tile kernel's above (the SwiGLU's 128-column
+// the decode tile kernel's at most 128 rows of X (the packed path's bits, and
+// its launch but where that is the small-M kernel's), the tile kernel's above (the SwiGLU's 128-column
 // plan, the matmul's accumulating plan, and their bits; K a multiple of 64,
 // N of 8); otherwise each call packs wg
 // and wu into the MFMA operand layout on the device (one pack launch per

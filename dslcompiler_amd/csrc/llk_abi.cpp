@@ -963,10 +963,9 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
   if (M <= 64 && llk::tunable("flex_tile") <= 1) {
     // The decode tile kernel unsplit, narrower outputs (N <= 2176) and calls for
     // which a knob or a schedule record has chosen keep their plans, which
-    // callers and tests hold this library to; row-major weights have no small-M
-    // form.
+    // callers and tests hold this library to.
     llk::ScheduleEntry se;
-    if (!x || rowmajor || NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws ||
+    if (!x || NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws ||
         llk::tunable("flex_tile") == 0 || llk::tunable("decode_max_m") != 64 || llk::tunable("decode_splits") > 0 ||
         llk::tunable("decode_group_width") > 0 || llk::tunable("decode_tile") != 1 ||
         llk::tunable("decode_target_wgs") != 256 || llk::tunable("decode_min_kb") != 2 ||
@@ -975,7 +974,20 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     const Plan ref = max_ws != SIZE_MAX
                          ? plan_launch_large(nmat, M, K, KB, NB, x, SIZE_MAX, accumulate, out_bf16)
                          : p;
-    return small_plan(p, ref, nmat, M, K, KB, NB, x);
+    const Plan q = small_plan(p, ref, nmat, M, K, KB, NB, x);
+    if (!rowmajor) return q;
+    // Row-major weights have no small-M form (those the decode tile kernel
+    // cannot read are packed, and take q): the decode tile kernel with that
+    // kernel's k parts as its splits.  Both run the same MFMAs over each part
+    // and add the parts in order, so the result is the packed call's bit for
+    // bit.  It costs a synchronous KernelFn call 14% in the mean of 36 shapes
+    // (M = 7, K = 1728, N = 3456 23.7 -> 26.3 us in 7 splits for 4).
+    if (p.dtile && q.skinny && !q.dtile) {
+      const int64_t part = chain_steps(q, nmat, M, KB);
+      p.S = (int)((KB + part - 1) / part);
+      p.ws_bytes = p.need = llk_skinny_workspace_bytes(nmat, (int)M, (int)(NB * 128), p.S);
+    }
+    return p;
   }
   const int64_t knob = llk::tunable("flex_tile");
   const int64_t forced_s = llk::tunable("tile_splits");
@@ -1857,7 +1869,9 @@ int pack_into(const llk_tensor2d* w, int64_t bk, bool w_on_device, void* dst, hi
 //  * the dispatcher's plan for the shape and X is the decode tile kernel
 //    with at most 128 rows and the weights' rows suit its loads
 //    (llk_decode_rowmajor_fits): that plan, with the same grid, k splits and
-//    MFMA operands, so the result equals the packed path's bit for bit;
+//    MFMA operands, so the result equals the packed path's bit for bit; up to
+//    64 rows, where the packed path may take the small-M kernel in one launch
+//    instead, the splits are that kernel's k parts, with the same bits;
 //  * otherwise, on the tile path (X aligned, K a multiple of 64,
 //    llk_tile_rowmajor_fits), the tile kernel's row-major form: for the
 //    fused SwiGLU (bf16 or fp32 result), the 128-column kernel's plan -- k

@@ -292,6 +292,53 @@ def test_kernel_fn_rowmajor_matches_packed(llk, gpu, orc, M, K, N, ldw):
     assert_parity_bf16(got, orc.swiglu(x, wg, wu)[0], f"KernelFn row-major M={M}")
 
 
+# One shape per small-M form that the packed path takes in place of a k split
+# (N > 2176): operation, rows above 32 or not, 32-column groups per workgroup.
+ONE_LAUNCH = [(0, 26, 576, 2184, 1), (0, 11, 1728, 8200, 2), (0, 54, 704, 2184, 1),
+              (0, 1, 640, 2304, 1), (3, 17, 512, 2184, 1), (3, 27, 1152, 2184, 2),
+              (3, 37, 576, 2208, 1), (3, 42, 896, 8200, 2)]
+
+
+@pytest.mark.parametrize("op,M,K,N,W", ONE_LAUNCH)
+def test_kernel_fn_rowmajor_matches_one_launch_plan(llk, gpu, tile_knobs, op, M, K, N, W):
+    """Up to 64 rows where the packed call runs the small-M kernel in one
+    launch: the row-major KernelFn, which has the decode tile kernel alone,
+    gives the packed call's bits, as do a call that packs and (SwiGLU) one
+    that reuses packed weights."""
+    print(f"case kernel_fn one launch op={op} M={M} K={K} N={N}", flush=True)
+    plan = llk.describe_launch("fused_swiglu" if op == 0 else "matmul", M, N, K,
+                               accumulate=op == 3)
+    assert (plan["kernel"], plan["splits"], plan["group_width"]) == ("small_m", 1, W), plan
+    x, wg, wu = swiglu_inputs(M, K, N, seed=M + N)
+    xd, wgd, wud = to_dev(gpu, x), to_dev(gpu, wg), to_dev(gpu, wu)
+    pg, pu = llk.PackedWeights.from_host(wg), llk.PackedWeights.from_host(wu)
+    jc = llk.JitCache()
+    fn = jc.lookup_or_compile(llk.KernelKey(operation=op, isa=7, N=N, K=K, output_type=2))
+    init = gpu.randn((M, N), dtype=gpu.float32, device="cuda")
+    if op == 0:
+        want = from_dev(llk.fused_swiglu(xd, pg, pu, out_dtype=gpu.float32))
+    else:
+        want = from_dev(llk.matmul(xd, pg, out=init.clone(), accumulate=True))
+    for on in (1, 0):
+        tile_knobs(kernel_fn_rowmajor=on)
+        y = gpu.full((M, N), float("nan"), dtype=gpu.float32, device="cuda")
+        fn(xd, wgd, wud if op == 0 else None, init, y)
+        assert np.array_equal(from_dev(y), want), f"kernel_fn_rowmajor={on}"
+    jc.close()
+    if op == 0:
+        y = gpu.full((M, N), float("nan"), dtype=gpu.bfloat16, device="cuda")
+        L = llk.lib()
+        assert L.llk_kernel_fn_assume_immutable_weights(1) == 0
+        try:
+            L.llk_cache_clear(L.llk_kernel_fn_cache())  # no entry at a reused address
+            _call(llk, _memref(xd.data_ptr(), M, K, K), _memref(wgd.data_ptr(), K, N, N),
+                  _memref(wud.data_ptr(), K, N, N), _memref(y.data_ptr(), M, N, N))
+        finally:
+            assert L.llk_kernel_fn_assume_immutable_weights(0) == 1
+            L.llk_cache_clear(L.llk_kernel_fn_cache())
+        assert np.array_equal(from_dev(y), from_dev(llk.fused_swiglu(xd, pg, pu)))
+
+
 @pytest.mark.parametrize("M,S", [(8, 0), (40, 3), (100, 0), (200, 0), (600, 0), (300, 5)])
 def test_kernel_fn_rowmajor_matmul_entry(llk, gpu, orc, M, S):
     """The object-code level's matmul KernelFn (fp32 key, result = init + x
