@@ -1019,13 +1019,10 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     // X rows that start inside a 128-byte line (whose lines are read twice)
     // slow a step by 8%, rows off the 16 bytes by 20% and at odd elements by
     // 25% (K = 1600 against 1599 and 1598, N = 4288, M = 3779: 60.8, 67.1 and
-    // 67.4 us with the larger tiles, 18.2 to 20.1 us at M = 400).
+    // 67.4 us with the larger tiles, 18.2 to 20.1 us at M = 400).  Told from K,
+    // the stride of dense rows: a view's own stride must not change the sums.
     const bool aligned = x && x_vec_ok(x);
-    const double slow =
-        !x ? 1.0
-           : aligned ? (x->stride0 % 64 != 0 ? 1.08 : 1.0)
-                     : (x->stride0 | (int64_t)(reinterpret_cast<uintptr_t>(x->data) / 2)) & 1 ? 1.25
-                                                                                              : 1.20;
+    const double slow = aligned ? (K % 64 != 0 ? 1.08 : 1.0) : (K & 1 ? 1.25 : 1.20);
     // taken when modelled 5% faster; 12% on rows off the 16 bytes, where the
     // two models are rougher
     double best = (aligned ? 0.95 : 0.88) * plan_us(ref, nmat, M, KB, NB);

@@ -66,3 +66,25 @@ def test_ragged_k_any_alignment(llk, gpu, M, K):
         want = from_dev(llk.matmul(to_dev(gpu, xp), pp))
         for off, pad in ((0, 0), (0, 1), (1, 3)):
             assert np.array_equal(from_dev(llk.matmul(_at(gpu, x, off, pad), pg)), want), (off, pad)
+
+
+# The launch depends on the shape and on whether X's rows are 16-byte aligned;
+# views of one alignment then take the same sums.
+STRIDED = [("matmul", 219, 640, 517), ("fused_swiglu", 101, 2752, 860),
+           ("fused_swiglu", 117, 732, 533), ("matmul", 195, 583, 718)]
+
+
+@pytest.mark.parametrize("op,M,K,N", STRIDED)
+def test_row_stride_leaves_the_sums_alone(llk, gpu, op, M, K, N):
+    print(f"case row stride {op} M={M} K={K} N={N}", flush=True)
+    x, wg, wu = swiglu_inputs(M, K, N, seed=M + K)
+    pg, pu = llk.PackedWeights.from_host(wg), llk.PackedWeights.from_host(wu)
+    views = ((0, 0), (0, 8), (8, 56)) if K % 8 == 0 else ((0, 0), (0, 1), (1, 0), (1, 2), (2, 0))
+    got = []
+    for off, pad in views:
+        xd = _at(gpu, x, off, pad)
+        y = llk.matmul(xd, pg) if op == "matmul" else llk.fused_swiglu(xd, pg, pu,
+                                                                      out_dtype=gpu.float32)
+        got.append(from_dev(y))
+    for g, v in zip(got, views):
+        assert np.array_equal(g, got[0]), v
