@@ -943,9 +943,10 @@ Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, 
 }
 
 // The plan: above 64 rows the flex tile kernel where it is modelled faster.
-// The choice depends on the shape and X's alignment alone -- not on the
-// result type or on the workspace at hand -- so a bf16 result stays the
-// rounding of the fp32 one.
+// The choice depends on the shape and X's alignment, not on the result type, so
+// a bf16 result stays the rounding of the fp32 one.  Where a caller's scratch
+// holds the plan without this kernel's planes but not with them (below what
+// llk_swiglu_scratch_size and llk_describe_launch answer), that plan runs.
 // Kept on the other kernels: 512 or fewer k, 768 or fewer for C += A B (the
 // launches and scratch of such plans are part of what callers and tests hold
 // this library to), X at an odd base or row stride (K itself a
@@ -953,8 +954,7 @@ Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, 
 // than 128 MB of weights (the k loop then streams from HBM; of ten shapes
 // measured there this kernel was 6 and 9% faster on two and 5 to 33% slower on
 // the others), X beyond one launch's 32-bit offsets, and every call for which a knob or a schedule
-// record has chosen among those kernels.  A caller's scratch (max_ws) that
-// holds the other plan but not this one's planes gets the other plan.
+// record has chosen among those kernels.
 Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const llk_tensor2d* x,
                  size_t max_ws = SIZE_MAX, bool accumulate = false, bool out_bf16 = true,
                  bool rowmajor = false) {
@@ -965,7 +965,7 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     // which a knob or a schedule record has chosen keep their plans, which
     // callers and tests hold this library to.
     llk::ScheduleEntry se;
-    if (!x || NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws ||
+    if (NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws ||
         llk::tunable("flex_tile") == 0 || llk::tunable("decode_max_m") != 64 || llk::tunable("decode_splits") > 0 ||
         llk::tunable("decode_group_width") > 0 || llk::tunable("decode_tile") != 1 ||
         llk::tunable("decode_target_wgs") != 256 || llk::tunable("decode_min_kb") != 2 ||
@@ -1021,7 +1021,7 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     // 25% (K = 1600 against 1599 and 1598, N = 4288, M = 3779: 60.8, 67.1 and
     // 67.4 us with the larger tiles, 18.2 to 20.1 us at M = 400).  Told from K,
     // the stride of dense rows: a view's own stride must not change the sums.
-    const bool aligned = x && x_vec_ok(x);
+    const bool aligned = x_vec_ok(x);
     const double slow = aligned ? (K % 64 != 0 ? 1.08 : 1.0) : (K & 1 ? 1.25 : 1.20);
     // taken when modelled 5% faster; 12% on rows off the 16 bytes, where the
     // two models are rougher
@@ -1047,13 +1047,9 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
       }
     }
   }
-  if (!cfg || (x && !llk_flex_fits(M, K, x->stride0, 0, 0))) return p;
+  if (!cfg || !llk_flex_fits(M, K, x->stride0, 0, 0)) return p;
   const size_t bytes = S > 1 ? (size_t)S * nmat * M * NB * 512 : 0;
   if (bytes > max_ws) return p;
-  if (!x) {  // sizing: whichever needs more
-    p.ws_bytes = std::max(p.ws_bytes, bytes);
-    return p;
-  }
   Plan q;
   q.flex = cfg;
   q.S = (int)S;
@@ -1582,13 +1578,27 @@ int llk_packed_weights_load(const char* path, unsigned flags, llk_packed_weights
 // Kernels
 // ---------------------------------------------------------------------------
 
+// An X with the given alignment for plan_launch, which reads only the
+// pointer's alignment, the row stride and the shape.
+static llk_tensor2d stand_in_x(int64_t M, int64_t K, bool aligned) {
+  return {reinterpret_cast<void*>(aligned ? 256 : 2), M, K, aligned ? K : K + 1, 1};
+}
+
 size_t llk_swiglu_scratch_size(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   // Either output type (the bf16 plan may take the wide kernel, which needs
-  // no partial planes).
+  // no partial planes), X at either alignment or in need of a padded copy.
   const int64_t KB = llk::deviceBlocksK(K), NB = llk::deviceBlocksN(N);
-  return std::max(plan_launch(2, M, K, KB, NB, nullptr, SIZE_MAX, false, true).ws_bytes,
-                  plan_launch(2, M, K, KB, NB, nullptr, SIZE_MAX, false, false).ws_bytes);
+  size_t bytes = 0;
+  for (const bool bf16 : {true, false}) {
+    bytes = std::max(
+        bytes, plan_launch_large(2, M, K, KB, NB, nullptr, SIZE_MAX, false, bf16).ws_bytes);
+    for (const bool aligned : {true, false}) {
+      const llk_tensor2d x = stand_in_x(M, K, aligned);
+      bytes = std::max(bytes, plan_launch(2, M, K, KB, NB, &x, SIZE_MAX, false, bf16).ws_bytes);
+    }
+  }
+  return bytes;
 }
 
 int llk_describe_launch(int operation, int64_t M, int64_t N, int64_t K, unsigned flags,
@@ -1606,10 +1616,7 @@ int llk_describe_launch(int operation, int64_t M, int64_t N, int64_t K, unsigned
     return fail(LLK_ERR_SHAPE, "M, N, K must be in [1, 2^30]");
   const int nmat = operation == 0 ? 2 : 1;
   const int64_t KB = llk::deviceBlocksK(K), NB = llk::deviceBlocksN(N);
-  // A stand-in X with the requested alignment (plan_launch reads only the
-  // pointer's alignment, the row stride and K).
-  const bool x_aligned = (flags & LLK_PLAN_X_ALIGNED) != 0;
-  llk_tensor2d x{reinterpret_cast<void*>(x_aligned ? 256 : 2), M, K, x_aligned ? K : K + 1, 1};
+  const llk_tensor2d x = stand_in_x(M, K, (flags & LLK_PLAN_X_ALIGNED) != 0);
   const Plan p = plan_launch(nmat, M, K, KB, NB, &x, SIZE_MAX, accumulate,
                              (flags & LLK_PLAN_OUT_F32) == 0);
   if (p.too_large)

@@ -36,3 +36,19 @@ def test_sums_no_longer(op, rows):
         finally:
             llk.set_tunable("flex_tile", 1)
         assert _longest(new, op, M, K) <= _longest(old, op, M, K), (op, M, K, N, new, old)
+
+
+def test_scratch_size_covers_every_plan():
+    """A caller who sizes scratch with the library's own query has room for
+    the launch the library takes, for either result type and alignment of X."""
+    rng = random.Random(4)
+    shapes = [(713, 3384, 1325), (547, 3984, 1330), (265, 3648, 676), (192, 4928, 839)]
+    for _ in range(400):
+        K, N = rng.randint(512, 6000), rng.randint(512, 3000)
+        shapes.append((rng.randint(1, 800), K - K % rng.choice([1, 8, 64]), N))
+    for M, K, N in shapes:
+        size = llk.swiglu_scratch_size(M, N, K)
+        for aligned in (True, False):
+            for f32 in (True, False):
+                plan = llk.describe_launch("fused_swiglu", M, N, K, x_aligned=aligned, out_f32=f32)
+                assert plan["workspace_bytes"] <= size, (M, K, N, aligned, f32, plan, size)
