@@ -208,10 +208,12 @@ bool capturing(hipStream_t s) {
 }
 
 // Evicts the least recently used idle, unpinned workspace of `st` other
-// than `keep`; false if there is none, or if the device cannot be waited for
-// (a graph is being captured).  Its stream may be gone, with work still
-// queued, so the whole device is waited for: eviction is rare.  Called with
-// the device mutex held.
+// than `keep`; false if there is none, or if it cannot be freed now (a graph
+// is being captured in the global mode).  hipFree waits for the device, so
+// work still queued, also on a stream that is gone, has finished with the
+// buffer.  (A wait of our own, hipDeviceSynchronize, would break a capture
+// under way in another thread whatever its mode.)  Called with the device
+// mutex held.
 bool evict_one_workspace(DeviceState& st, const Workspace* keep) {
   auto victim = st.ws.end();
   for (auto it = st.ws.begin(); it != st.ws.end(); ++it) {
@@ -220,12 +222,9 @@ bool evict_one_workspace(DeviceState& st, const Workspace* keep) {
     if (victim == st.ws.end() || w.tick < victim->second.tick) victim = it;
   }
   if (victim == st.ws.end()) return false;
-  if (victim->second.ptr) {
-    if (hipDeviceSynchronize() != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    (void)hipFree(victim->second.ptr);
+  if (victim->second.ptr && hipFree(victim->second.ptr) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
   }
   st.ws.erase(victim);
   return true;
@@ -239,12 +238,12 @@ bool evict_one_workspace(DeviceState& st, const Workspace* keep) {
 // on the capture stream is the caller's race, as with any captured buffer.)
 // The library keeps at most `max_workspaces` of them per device (tunable,
 // default 16): a new stream (or thread, on the per-thread default stream)
-// beyond that evicts the least recently used idle one.  A buffer is freed on
-// growth only after its stream, and on eviction or by llk_workspace_trim only
-// after the device, has been waited for, so work still queued -- even on a
-// stream destroyed since -- never loses its buffer, and no call pays for an
-// event of its own (naming one as a kernel's stop event cost 4 us a launch on
-// the host: two launches 11.6 -> 6 us).  A workspace that a call used while its
+// beyond that evicts the least recently used idle one.  A buffer is freed (on
+// growth, on eviction or by llk_workspace_trim) with hipFree, which waits for
+// the device, so work still queued -- even on a stream destroyed since --
+// never loses its buffer, and no call pays for an event of its own (naming
+// one as a kernel's stop event cost 4 us a launch on the host: two launches
+// 11.6 -> 6 us).  A workspace that a call used while its
 // stream was capturing a graph is pinned instead (the graph names it) and is
 // never freed.  Growth is geometric (x1.5 at least).  *held is the library
 // workspace handed out (null for a caller's scratch or when nothing is
@@ -282,10 +281,7 @@ int get_workspace(int dev, size_t need, size_t asked, llk_kernel_context* ctx, v
   if (w->bytes < need) {
     const size_t bytes = std::max({need, w->bytes + w->bytes / 2, (size_t)1 << 20});
     if (w->ptr) {
-      const hipStream_t s = ctx ? static_cast<hipStream_t>(ctx->stream) : nullptr;
-      if (!w->pinned && w->busy == 0 && !capturing(s) && hipStreamSynchronize(s) == hipSuccess) {
-        (void)hipFree(w->ptr);  // this stream's earlier calls have finished with it
-      } else {
+      if (w->pinned || w->busy > 0 || hipFree(w->ptr) != hipSuccess) {
         (void)hipGetLastError();
         try {
           st.retired.push_back(w->ptr);  // a graph or a concurrent call may still name it

@@ -259,3 +259,70 @@ def test_accumulate_scratch_sized_from_plan(llk, gpu, orc):
     small = gpu.empty(plan["workspace_bytes"] - 256, dtype=gpu.uint8, device="cuda")
     with pytest.raises(llk.LLKError, match="SCRATCH"):
         llk.matmul(xd, pb, out=c0.clone(), accumulate=True, scratch=small)
+
+
+@pytest.mark.parametrize("mode", ["thread_local", "relaxed"])
+def test_trim_while_another_thread_captures(llk, gpu, orc, mode):
+    """llk_workspace_trim from a second thread while a graph is captured: the
+    idle workspaces are freed once the work queued on them is done, and the
+    capture, whose own workspace is in use, ends and replays as without it."""
+    import ctypes as C
+    import threading
+    from dslcompiler_amd._lib import KernelContext, tensor2d
+    print(f"case trim during capture {mode}", flush=True)
+    M, K, N = 300, 2048, 640
+    x, wg, wu = swiglu_inputs(M, K, N, seed=95)
+    pg, pu = llk.PackedWeights.from_host(wg), llk.PackedWeights.from_host(wu)
+    xd = to_dev(gpu, x)
+    ref = orc.swiglu(x, wg, wu)[0]
+    y_cap, y_side = (gpu.empty((M, N), dtype=gpu.bfloat16, device="cuda") for _ in range(2))
+    cap, side = gpu.cuda.Stream(), gpu.cuda.Stream()
+    L = llk.lib()
+
+    def call(stream, y):
+        ctx = KernelContext(None, 0, stream.cuda_stream)
+        rc = L.llk_swiglu_bf16(C.byref(tensor2d(xd.data_ptr(), M, K)), pg.handle, pu.handle,
+                               C.byref(tensor2d(y.data_ptr(), M, N)), 0, C.byref(ctx))
+        assert rc == 0, L.llk_last_error()
+
+    old = llk.get_tunable("tile_splits")
+    llk.set_tunable("tile_splits", 3)  # partial planes: a workspace per stream
+    gpu.cuda.synchronize()
+    try:
+        llk.workspace_trim()
+        kept = llk.workspace_stats()[0]  # pinned by graphs of earlier tests
+        for s, y in ((cap, y_cap), (side, y_side)):
+            call(s, y)
+        gpu.cuda.synchronize()
+        eager = from_dev(y_cap)
+        seen = {}
+
+        def trim():
+            for _ in range(400):  # about 10 ms of work queued on the side stream
+                call(side, y_side)
+            done = gpu.cuda.Event()
+            done.record(side)
+            seen["before"] = done.query()
+            llk.workspace_trim()
+            seen["after"] = done.query()
+            seen["left"] = llk.workspace_stats()[0]
+
+        g = gpu.cuda.CUDAGraph()
+        with gpu.cuda.graph(g, stream=cap, capture_error_mode=mode):
+            call(cap, y_cap)
+            t = threading.Thread(target=trim)
+            t.start()
+            t.join()
+        assert seen == {"before": False, "after": True, "left": kept + 1}, seen
+        assert_parity_bf16(from_dev(y_side), ref, "side stream")
+        for rep in range(3):
+            y_cap.zero_()
+            gpu.cuda.synchronize()
+            g.replay()
+            gpu.cuda.synchronize()
+            assert np.array_equal(from_dev(y_cap), eager), rep
+            call(side, y_side)  # a fresh workspace after the trim
+            gpu.cuda.synchronize()
+            assert np.array_equal(from_dev(y_side), eager)
+    finally:
+        llk.set_tunable("tile_splits", old)
