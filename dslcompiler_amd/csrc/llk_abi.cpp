@@ -759,30 +759,44 @@ Plan plan_launch_large(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
 
 // The flex tile kernel (kernels/flex_tile.hip) against the plan above it.
 // Both times are modelled in microseconds, fitted on MI355X measurements of
-// 370 random shapes (M 65..4097, K 512..13824, N 512..14336, both operations;
-// each model within 4-10% rms, the tile kernel's unsplit one 15%).  Over them
-// the choice the models make runs 1.42x the plan without this kernel in the
-// geometric mean, always taking the fastest measured 1.43x, both before the
-// limit of chain_steps on the sums' length.
-//   us = a + b n kbs + c kbs + d (MB of Y, or of planes when S > 1)
-//          + e (MB of weights) + f n + g (MB of weights beyond 80)
+// 5000 random shapes (M 65..4097, K 576..13824, N 512..14336, both operations)
+// whose weights come from HBM, as they do between the layers of a model: each
+// model within 6-7% rms.  (Fitted on weights that stay in cache, as before,
+// the models took this kernel at 330 of the 5000 that run over 3% slower with
+// it, by up to 26%: C = A B 3501 x 640 x 12384 70.5 us without it, 95.7 with,
+// SwiGLU 74 x 896 x 11104 12.5 and 15.7 us.)  Over them the choice runs 1.165x
+// the plan without this kernel in the geometric mean, the fastest measured
+// 1.171x; where it differs (2527) 1.35x, at 26 over 3% slower.
+//   us = base + slow kbs step[n] + out (MB of Y, or of planes when S > 1)
+//          + weights (MB of weights)
 // with n = ceil(workgroups / 256) and kbs = 64-k steps per split: the
 // smaller tiles pay less for a short grid or a ragged edge, the larger ones
-// less per multiply-add.
+// less per multiply-add; two or more workgroups on a CU hide each other's
+// loads, so step grows less than n.  (M x K x N.)
+struct FlexCost {
+  double base, step[4];  // n = 1..4; beyond, in proportion to the last
+  double out, weights;
+  double us(int64_t n, int64_t kbs, double out_mb, double w_mb, double slow) const {
+    return base + slow * (double)kbs * (n < 4 ? step[n - 1] : step[3] * (double)n / 4.0) +
+           out * out_mb + weights * w_mb;
+  }
+};
 struct FlexModel {
   int cfg, tm, tn;  // tile: rows, MFMA rows
-  double one[7], many[7];
+  FlexCost one, many;
 };
 constexpr FlexModel kFlex[] = {
-    {222, 64, 64, {2.87, 0.197, 0.044, 0.124, 0, 0.30, 0.117},
-     {6.3, 0.090, 0.162, 0.453, 0.0065, 0.69, 0.655}},
-    {224, 64, 128, {3.46, 0.283, 0.040, 0.169, 0.010, 0.29, 0.146},
-     {7.4, 0.177, 0.142, 0.324, 0.002, 0.75, 0.204}},
-    {244, 128, 128, {3.89, 0.402, 0, 0.192, 0.0076, 0.89, 0.166},
-     {9.5, 0.349, 0, 0.307, 0.021, 0, 0.146}},
+    {222, 64, 64, {2.69, {0.360, 0.515, 0.720, 0.910}, 0.136, 0.048},
+     {6.69, {0.015, 0.231, 0.405, 0.514}, 0.570, 0.110}},
+    {224, 64, 128, {2.94, {0.391, 0.621, 0.884, 1.239}, 0.194, 0.084},
+     {8.23, {0.000, 0.402, 0.602, 0.850}, 0.392, 0.109}},
+    {244, 128, 128, {3.75, {0.485, 0.844, 1.329, 1.841}, 0.231, 0.077},
+     {9.37, {0.272, 0.747, 1.212, 1.671}, 0.280, 0.096}},
 };
 
-// Modelled microseconds of a plan of the other kernels above 64 rows.
+// Modelled microseconds of a plan of the other kernels above 64 rows, fitted
+// on the same measurements (decode tile kernel within 5% rms, the tile kernels
+// 6-7%; none of them has an unsplit head, whose term is an earlier fit's).
 double plan_us(const Plan& p, int nmat, int64_t M, int64_t KB, int64_t NB) {
   const double y_mb = M * NB * 128 * 3e-6, w_mb = KB * NB * 16384e-6 * nmat;
   const double past = std::max(0.0, w_mb - 80.0);
@@ -791,25 +805,25 @@ double plan_us(const Plan& p, int nmat, int64_t M, int64_t KB, int64_t NB) {
   auto rounds = [](int64_t wgs) { return (double)((wgs + 255) / 256); };
   if (p.dtile) {
     const double t = rounds((nmat == 2 ? NB * 2 : NB) * p.S) * kbs;
-    return p.S > 1 ? 7.2 + 0.529 * t + 0.668 * planes + 0.002 * w_mb + 0.043 * past
-                   : 4.0 + 0.516 * t + 0.269 * y_mb + 0.024 * w_mb;
+    return p.S > 1 ? 6.67 + 0.482 * t + 0.715 * planes + 0.005 * w_mb + 0.033 * past
+                   : 4.25 + 0.501 * t + 0.329 * y_mb + 0.0195 * w_mb + 0.018 * past;
   }
   const int64_t tm = (M + 255) / 256;
   double us;
   if (p.wide && p.S == 1) {
     const double t = rounds(tm * ((NB * 8 + p.wide - 1) / p.wide)) * (kbs + 2) * p.wide / 8.0;
-    us = 3.2 + 1.22 * t + 0.266 * y_mb + 0.092 * past;
+    us = 4.70 + 1.131 * t + 0.314 * y_mb + 0.039 * past;
   } else {
     const int64_t per = nmat == 2 ? 1 : 2, tail = NB - p.head_nb;
     const double t =
         p.wide ? rounds(tm * ((NB * 8 + p.wide - 1) / p.wide) * p.S) * (kbs + 2) * p.wide / 8.0
                : rounds(tm * ((tail + per - 1) / per) * p.S) * (kbs + 2);
     const double part = (double)tail / NB;
-    us = p.S > 1 ? 13.4 + 1.044 * t + part * (0.208 * planes + 0.13 * past)
-                 : 1.8 + 1.096 * t + 0.356 * y_mb + 0.021 * w_mb + 0.033 * past;
+    us = p.S > 1 ? 10.24 + 1.101 * t + part * (0.214 * planes + 0.037 * past) + 0.030 * w_mb
+                 : 1.44 + 1.137 * t + 0.289 * y_mb + 0.011 * w_mb + 0.081 * past;
     if (p.head_nb > 0) us += 1.53 * rounds(tm * (p.head_nb / per)) * (KB + 2);
   }
-  if (p.pad) us += 3.0 + M * KB * 256 / 3e6;  // the padded copy of X
+  if (p.pad) us += 2.8 + M * KB * 37e-6;  // the padded copy of X
   return us;
 }
 
@@ -845,16 +859,11 @@ constexpr SmallModel kSmall[] = {
 };
 constexpr double kSmallDtile[2][7] = {{3.09, 0.366, 0, 0.024, 0.045, 2.11, 0.495},
                                       {3.53, 0.344, 0, 0.036, 0.015, 1.57, 0.451}};
-// The flex tile kernel unsplit at up to 64 rows (terms as in FlexModel).
+// The flex tile kernel unsplit at up to 64 rows and one 64-k step.
 constexpr FlexModel kSmallFlex[] = {
-    {222, 64, 64, {1.07, 0.025, 0.224, 0.663, 0.055, 1.69, 0.079}, {}},
-    {224, 64, 128, {3.17, 0.331, 0, 0.619, 0.045, 0, 0.117}, {}},
+    {222, 64, 64, {1.294, {1.715, 3.430, 5.145, 6.860}, 0.663, 0.055}, {}},
+    {224, 64, 128, {3.17, {0.331, 0.662, 0.993, 1.324}, 0.619, 0.045}, {}},
 };
-
-double flex_us(const double* c, double n, int64_t kbs, double out_mb, double w_mb, double slow) {
-  return c[0] + slow * c[1] * n * kbs + c[2] * kbs + c[3] * out_mb + c[4] * w_mb + c[5] * n +
-         c[6] * std::max(0.0, w_mb - 80.0);
-}
 
 // Small-M kernel: waves of a workgroup that share a column group's k.
 int small_m_k_waves(int nmat, int64_t M, int width) {
@@ -921,11 +930,11 @@ Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, 
     q = w;
     taken = true;
   }
-  if (KB <= longest && KB * NB * nmat <= 8192 && llk_flex_fits(M, K, x->stride0, 0, 0)) {
+  if (KB == 1 && NB * nmat <= 8192 && llk_flex_fits(M, K, x->stride0, 0, 0)) {
     const double y_mb = M * NB * 128 * 3e-6;
     for (const FlexModel& f : kSmallFlex) {
-      const double n = (double)((NB * 128 * nmat / f.tn + 255) / 256);
-      const double us = flex_us(f.one, n, KB, y_mb, w_mb, 1.0);
+      const int64_t n = (NB * 128 * nmat / f.tn + 255) / 256;
+      const double us = f.one.us(n, KB, y_mb, w_mb, 1.0);
       if (us >= best) continue;
       best = us;
       q = Plan{};
@@ -1019,9 +1028,7 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     // the stride of dense rows: a view's own stride must not change the sums.
     const bool aligned = x_vec_ok(x);
     const double slow = aligned ? (K % 64 != 0 ? 1.08 : 1.0) : (K & 1 ? 1.25 : 1.20);
-    // taken when modelled 5% faster; 12% on rows off the 16 bytes, where the
-    // two models are rougher
-    double best = (aligned ? 0.95 : 0.88) * plan_us(ref, nmat, M, KB, NB);
+    double best = 0.97 * plan_us(ref, nmat, M, KB, NB);
     if (!aligned && K % 8 == 0 && (M + 63) / 64 * (NB * 2 * nmat) < 128) return p;
     const double y_mb = M * NB * 128 * 3e-6, w_mb = KB * NB * 16384e-6 * nmat;
     for (const FlexModel& f : kFlex) {
@@ -1031,9 +1038,9 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
         if (want > 1 && (tiles * want > 1024 || KB / want < 3)) break;
         const int64_t kbs = (KB + want - 1) / want, s = (KB + kbs - 1) / kbs;
         if (kbs > longest) continue;
-        const double n = (double)((tiles * s + 255) / 256);
         const double us =
-            flex_us(s == 1 ? f.one : f.many, n, kbs,
+            (s == 1 ? f.one : f.many)
+                .us((tiles * s + 255) / 256, kbs,
                     s == 1 ? y_mb : s * nmat * M * NB * 512e-6, w_mb, slow);
         if (us < best) {
           best = us;

@@ -52,3 +52,22 @@ def test_scratch_size_covers_every_plan():
             for f32 in (True, False):
                 plan = llk.describe_launch("fused_swiglu", M, N, K, x_aligned=aligned, out_f32=f32)
                 assert plan["workspace_bytes"] <= size, (M, K, N, aligned, f32, plan, size)
+
+
+# (op, M, K, N, us with the other kernels, us with the flex tile kernel) on
+# MI355X, the weights from HBM at every call
+MEASURED = [
+    ("matmul", 3501, 640, 12384, 70.5, 95.7), ("matmul", 4061, 9896, 1696, 147.2, 190.4),
+    ("fused_swiglu", 110, 11904, 1488, 25.4, 33.8), ("matmul", 299, 3982, 11152, 53.6, 68.3),
+    ("fused_swiglu", 74, 896, 11104, 12.5, 15.7), ("matmul", 601, 4048, 5851, 49.0, 61.1),
+    ("fused_swiglu", 282, 8640, 976, 30.6, 35.8), ("fused_swiglu", 85, 704, 13280, 11.9, 14.8),
+    ("matmul", 4062, 546, 944, 24.4, 12.1), ("fused_swiglu", 860, 576, 2113, 20.3, 10.5),
+    ("matmul", 198, 1683, 848, 21.3, 11.5), ("fused_swiglu", 411, 896, 4432, 20.9, 13.6),
+    ("matmul", 926, 1946, 960, 30.0, 19.2), ("fused_swiglu", 300, 1000, 1100, 23.6, 15.1),
+]
+
+
+@pytest.mark.parametrize("op,M,K,N,other,flex", MEASURED)
+def test_flex_tile_kernel_where_it_is_faster(op, M, K, N, other, flex):
+    plan = llk.describe_launch(op, M, N, K, x_aligned=K % 8 == 0)
+    assert (plan["kernel"] == "flex_tile") == (flex < other), plan
