@@ -1,8 +1,9 @@
-"""Up to 64 rows with N > 2176: the one-launch kernels chosen in place of a k
-split (small-M unsplit at width 1 and 2, flex 64-row tiles), against the
-oracle on both sides of the rule, with every X alignment and output type, and
-the rule itself: the same kernel for every output type, workspace and for an
-accumulating call."""
+"""Up to 64 rows with N > 2176: the one-launch plans chosen in place of a k
+split (the small-M kernel unsplit at width 1 and 2) and, for K inside one
+64-k step, the flex tile kernel's 64-row tiles, against the oracle on both
+sides of the rule, with every X alignment and output type; and the rule
+itself: the same launch for every result type of the SwiGLU, and for C = A B
+and C += A B."""
 from __future__ import annotations
 
 import numpy as np
@@ -23,6 +24,10 @@ CASES = [
     ("fused_swiglu", 64, 2944, 576, True, "decode_tile", 1),
     ("fused_swiglu", 33, 4097, 1031, False, "small_m", 1),
     ("fused_swiglu", 41, 8496, 2241, False, "small_m", 1),
+    ("fused_swiglu", 64, 4096, 63, False, "flex_tile", 1),  # K inside one step
+    ("fused_swiglu", 54, 2184, 24, True, "flex_tile", 1),
+    ("matmul", 36, 8240, 10, False, "flex_tile", 1),
+    ("fused_swiglu", 64, 4096, 65, False, "small_m", 1),    # ... and one past it
 ]
 
 
@@ -56,9 +61,29 @@ def test_small_routes(llk, gpu, orc, op, M, N, K, aligned, kernel, S):
 def test_choice_ignores_type_and_accumulation(llk):
     for M in (1, 16, 33, 64):
         for N in (2177, 2560, 4097, 8496, 13824):
-            for K in (64, 520, 1031, 2048, 4096):
+            for K in (40, 64, 520, 1031, 2048, 4096):
                 al = K % 8 == 0
                 p = llk.describe_launch("matmul", M, N, K, x_aligned=al)
                 q = llk.describe_launch("matmul", M, N, K, x_aligned=al, accumulate=True)
+                r = llk.describe_launch("fused_swiglu", M, N, K, x_aligned=al)
+                s = llk.describe_launch("fused_swiglu", M, N, K, x_aligned=al, out_f32=True)
                 for k in ("kernel", "splits", "workgroups"):
                     assert p[k] == q[k], (M, N, K, p, q)
+                    assert r[k] == s[k], (M, N, K, r, s)
+
+
+def test_flex_choice_ignores_type(llk):
+    """Above 64 rows the other kernels' splits may differ by the SwiGLU's
+    result type (the wide tiles give bf16 alone); the flex tile kernel is
+    taken for both or neither, with one split."""
+    taken = 0
+    for M in (65, 128, 191, 300, 512, 1000):
+        for N in (544, 1100, 2048, 4432):
+            for K in (576, 1000, 1031, 2048, 4096):
+                p, q = (llk.describe_launch("fused_swiglu", M, N, K, x_aligned=K % 8 == 0,
+                                            out_f32=f32) for f32 in (False, True))
+                if "flex_tile" in (p["kernel"], q["kernel"]):
+                    taken += 1
+                    for k in ("kernel", "splits", "workgroups"):
+                        assert p[k] == q[k], (M, N, K, p, q)
+    assert taken > 20
