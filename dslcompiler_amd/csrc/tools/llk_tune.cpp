@@ -254,10 +254,14 @@ int main(int argc, char** argv) {
   for (int i = 0; i < count; ++i) {
     const auto& c = cands[i];
     const bool sm = c.plan.kernel == 0 || c.plan.kernel == 3;  // small-M or decode tile
+    // The flex tile kernel's rows, 64 or 128, from its grid.
+    const int64_t cols = std::max<int64_t>(1, c.plan.tile_columns);
+    const int64_t flex_rows =
+        c.plan.workgroups / c.plan.splits == (M + 63) / 64 * ((N + cols - 1) / cols) ? 64 : 128;
     // BM: rows per workgroup (the decode tile kernel: 64, or 128 / 256 at mid M)
     const int64_t BM = c.plan.kernel == 0   ? (M <= 32 ? 32 : 64)
                        : c.plan.kernel == 3 ? (M <= 64 ? 64 : M <= 128 ? 128 : 256)
-                       : c.plan.kernel == 4 ? (c.plan.tile_columns * nmat == 64 ? 64 : 128)
+                       : c.plan.kernel == 4 ? flex_rows
                                             : 256;
     // BN 0 / grain_size 0: the dispatcher chooses for each shape (for M <= 64
     // the decode tile kernel where it applies, else the small-M kernel's
@@ -272,7 +276,7 @@ int main(int argc, char** argv) {
                  "\"vector_width\": 8, \"num_threads\": %lld, \"parallel_axis\": \"%s\", "
                  "\"grain_size\": %d},\n     \"source\": \"llk-tune\", \"measured_us\": %.3f}%s\n",
                  op.c_str(), bucket, (long long)N, (long long)K, (long long)BM, (long long)BN,
-                 sm ? 64 : 32, sm ? 32 : 16, sm ? 32 : 16, (long long)c.plan.threads_per_workgroup, sm ? "n" : "mn", c.S, c.us,
+                 sm || c.plan.kernel == 4 ? 64 : 32, sm ? 32 : 16, sm ? 32 : 16, (long long)c.plan.threads_per_workgroup, sm ? "n" : "mn", c.S, c.us,
                  i + 1 < count ? "," : "");
   }
   std::fprintf(f, "  ]\n}\n");

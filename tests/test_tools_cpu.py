@@ -196,6 +196,21 @@ def test_tune_dry_run_writes_loadable_db(tmp_path):
     assert sel.BN == e["schedule"]["BN"] and sel.grain_size == e["schedule"]["grain_size"]
 
 
+@pytest.mark.parametrize("M,N,K,BM", [(96, 1376, 1536, 64), (96, 2048, 1536, 64),
+                                      (192, 1376, 2048, 128)])
+def test_tune_records_the_flex_tile(tmp_path, M, N, K, BM):
+    """The dispatcher's choice where that is the flex tile kernel (64 x 64,
+    64 x 128 and 128 x 128 MFMA rows, 64-k steps)."""
+    out = tmp_path / "tune.json"
+    r = subprocess.run([str(BIN / "llk-tune"), "--op=matmul", f"--M={M}", f"--N={N}", f"--K={K}",
+                        "--dry-run", f"-o={out}", "--top=1"],
+                       capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and "kernel=flex_tile" in r.stdout, r.stdout + r.stderr
+    e = json.loads(out.read_text())["entries"][0]["schedule"]
+    assert (e["BM"], e["BN"], e["BK"], e["grain_size"]) == (
+        BM, llk.describe_launch("matmul", M, N, K)["tile_columns"], 64, 0), e
+
+
 def test_tune_mid_m_candidates(tmp_path):
     """Mid M (the dispatcher's plan is the decode tile kernel's 128-row
     form): llk-tune's candidates are that kernel at decode_splits S, its
