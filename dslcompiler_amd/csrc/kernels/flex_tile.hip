@@ -4,13 +4,15 @@
 // SwiGLU), several workgroups per CU, any K, any alignment of X, of Y and of
 // row-major weights.
 //
-// What it replaces, at M = 300, K = 1000, N = 1100 (SwiGLU): a padded copy of
-// X, 72 workgroups of the 128-column kernel in four k splits and their reduce,
-// 27.8 us of kernels; here 175 workgroups in one launch, 8.3 us.  GEMM 924 x
-// 2560 x 3078: 38.2 -> 23.5 us; 579 x 1472 x 3760: 30.4 -> 15.6 us; SwiGLU 411
-// x 896 x 4432: 22.5 -> 14.5 us.  Where 256 x 256 tiles fill the chip they
-// stay ahead (GEMM 4096^3: 98 us against 139 us here): a 128 x 128 tile moves
-// twice the operand bytes per multiply-add.
+// Device time of the launches, weights from HBM, M x K x N, with the other
+// kernels and with this one as dispatched: GEMM 4062 x 546 x 944 24.6 -> 12.6 us
+// (one launch of 128 x 128 tiles for a padded copy of X and 64 workgroups of 256
+// x 256 tiles), SwiGLU 411 x 896 x 4432 20.8 -> 13.4 us (one launch), SwiGLU 300 x
+// 1000 x 1100 23.8 -> 15.4 us and GEMM 391 x 1440 x 2574 27.2 -> 20.0 us (four k
+// splits, as many as before, without the padded copy; the first unsplit, with
+// longer sums: 8.3 us).  Where 256 x 256 tiles fill the chip they stay ahead
+// (GEMM 4096^3: 98 us against 139 us here): a 128 x 128 tile moves twice the
+// operand bytes per multiply-add.
 //
 // Every operand goes memory -> registers -> LDS: a register load takes any
 // 2-byte aligned address, where an LDS-DMA load needs aligned rows, and the
@@ -58,14 +60,14 @@ struct FlexCfg {
   static constexpr int XOFF = TN * 128;             // X behind the weights in a slot
   static constexpr int SLOT = (TN + TM) * 128;      // one 64-k step
   static constexpr int XL = TM / 32;                // 16-byte loads of X per thread and step
-  static constexpr int WL = (TN + 31) / 32;         // of W
+  static constexpr int WL = TN / 32;                // of W
   static constexpr int ROWB = WCOLS * 4 + 16;       // epilogue staging row
   // 64-k steps of loads in flight, in registers
   static constexpr int D = MI * NI <= 4 ? 3 : 2;
   // waves per SIMD (= workgroups per CU) the registers are kept to
   static constexpr int waves(bool rm) { return MI * NI <= 4 ? (rm ? 3 : 4) : MI * NI <= 8 ? 3 : 2; }
   static constexpr int LDS = 2 * SLOT > 64 * ROWB ? 2 * SLOT : 64 * ROWB;
-  static_assert(TM % 32 == 0 && NI % NMAT == 0, "tile");
+  static_assert(TM % 32 == 0 && TN % 32 == 0 && NI % NMAT == 0 && LDS <= 65536, "tile");
 };
 
 template <int NMAT, int WM, int MI, int NI, bool SPLIT, bool RM>
@@ -161,7 +163,6 @@ __global__ __launch_bounds__(256, (FlexCfg<NMAT, WM, MI, NI>::waves(RM))) void f
       wcols[q] = a.N - col;
     }
   }
-  constexpr bool kAllW = C::TN % 32 == 0;  // every wave moves WL operands
   auto load_w = [&](int kb, u32x4 (&wr)[WL]) {
 #pragma unroll
     for (int q = 0; q < WL; ++q) {
@@ -187,8 +188,7 @@ __global__ __launch_bounds__(256, (FlexCfg<NMAT, WM, MI, NI>::waves(RM))) void f
   auto write_w = [&](int slot, const u32x4 (&wr)[WL]) {
 #pragma unroll
     for (int q = 0; q < WL; ++q)
-      if (kAllW || q * 4 + wave < C::TN / 8)
-        *reinterpret_cast<u32x4*>(smem + slot * C::SLOT + wlds[q]) = wr[q];
+      *reinterpret_cast<u32x4*>(smem + slot * C::SLOT + wlds[q]) = wr[q];
   };
   auto write_x = [&](int slot, const u32x4 (&xr)[XL]) {
 #pragma unroll
@@ -467,17 +467,11 @@ template <int NMAT, int WM, int MI, int NI, bool SPLIT, bool RM>
 static hipError_t launch_flex_t(FlexArgs& a, const llk::ModuleFns* mod, hipStream_t s) {
   auto fn = flex_tile_kernel<NMAT, WM, MI, NI, SPLIT, RM>;
   using C = FlexCfg<NMAT, WM, MI, NI>;
-  constexpr int kLds = C::LDS;
-  if (kLds > 65536 && !mod) {
-    static std::atomic<uint64_t> lds_set{0};
-    hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), kLds, lds_set);
-    if (e != hipSuccess) return e;
-  }
   a.tiles_m = (a.M + C::TM - 1) / C::TM;
   a.tiles_n = (a.N + C::COLS - 1) / C::COLS;
   a.group_m = 2048 / C::TM;
   return launch_kernel(mod, reinterpret_cast<const void*>(fn), &flex_tile_symbol<NMAT, WM, MI, NI, SPLIT, RM>,
-                       dim3((unsigned)(a.tiles_m * a.tiles_n * a.S)), dim3(256), kLds, s, a);
+                       dim3((unsigned)(a.tiles_m * a.tiles_n * a.S)), dim3(256), C::LDS, s, a);
 }
 
 template <int NMAT, int WM, int MI, int NI, bool RM>

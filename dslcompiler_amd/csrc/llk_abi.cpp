@@ -827,22 +827,25 @@ double plan_us(const Plan& p, int nmat, int64_t M, int64_t KB, int64_t NB) {
   return us;
 }
 
-// Up to 64 rows, one launch instead of the decode tile kernel's (or the small-M
-// kernel's) k split and reduce, or the small-M kernel's for K inside a 64-k step:
-// the small-M kernel unsplit at width 1 or 2, whose waves split k inside a
-// workgroup, or the flex tile kernel's 64-row tiles.  Microseconds, fitted on
-// 420 random shapes (M 1..64, K 512..13824, N 512..14336) within 4-7% rms, the
-// decode tile kernel 10%:
+// Up to 64 rows, one launch instead of the decode tile kernel's (seldom the
+// small-M kernel's) k split and reduce: the small-M kernel unsplit at width 1 or
+// 2, whose waves split k inside a workgroup.  For K inside one 64-k step, where
+// nothing is split, the flex tile kernel's 64-row tiles instead of the small-M
+// kernel.  Microseconds, fitted on 420 random shapes (M 1..64, K 512..13824, N
+// 512..14336) within 4-7% rms, the decode tile kernel 10%:
 //   small-M      c0 + c1 s + c2 W/2 r kbs + c3 r + c4 (MB of weights)
 //                  + (c5, X aligned, or c6) r kbs X + S > 1: c7 + c8 (MB of planes)
 //   decode tile  c0 + c1 r kbs + c3 (MB of weights) + c4 (MB beyond 80)
 //                  + S > 1: c5 + c6 (MB of planes)
 // with r = ceil(workgroups / 256), kbs = 64-k steps per split, s = steps per
 // wave and X = M / 32 times the wave groups that read it.  A second launch costs
-// the host too: 1 us.  Over the 296 shapes with N > 2176 the choice is 1.11x
-// the plan without it in the geometric mean of device time; M x N x K: GEMM
-// 2 x 2648 x 640 6.8 -> 3.9 us, 56 x 8560 x 4035 41.4 -> 23.7 us, SwiGLU
-// 2 x 7163 x 1920 13.2 -> 11.4 us; none lost (before the limit of chain_steps).
+// the host too: 1 us.  Device time over 1200 other shapes with N > 2176, weights
+// from HBM: 1.098x the plan without this choice in the geometric mean (always
+// taking the fastest 1.100x); where it differs (481) 1.26x, at 6 over 3% slower
+// (by 7% at most).  M x K x N: GEMM 2 x 640 x 2648 6.9 -> 4.0 us, 29 x 1216 x
+// 7824 10.9 -> 7.5 us, SwiGLU 2 x 1920 x 7163 14.4 -> 11.8 us.  K below 64: 21 of
+// 400 shapes take the flex tile kernel, 1.36x, none slower (SwiGLU 64 x 63 x 4096
+// 5.5 -> 4.2 us).
 struct SmallModel {
   int nmat, mt, width;
   double c[9];
@@ -915,7 +918,7 @@ Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, 
   } else {
     best = small_m_us(ref.G, ref.S, aligned, nmat, M, KB, NB);
   }
-  // Below these margins the fit's own error chose: 7 of 296 lost 2-10%.
+  // Margins against the fit's own error (losses without them: 2-10%).
   best = ref.S > 1 ? 0.96 * (best + 1.0) : 0.86 * best;
   Plan q;
   bool taken = false;
@@ -948,27 +951,33 @@ Plan small_plan(const Plan& p, const Plan& ref, int nmat, int64_t M, int64_t K, 
 }
 
 // The plan: above 64 rows the flex tile kernel where it is modelled faster.
-// The choice depends on the shape and X's alignment, not on the result type, so
-// a bf16 result stays the rounding of the fp32 one.  Where a caller's scratch
-// holds the plan without this kernel's planes but not with them (below what
-// llk_swiglu_scratch_size and llk_describe_launch answer), that plan runs.
-// Kept on the other kernels: 512 or fewer k, 768 or fewer for C += A B (the
-// launches and scratch of such plans are part of what callers and tests hold
-// this library to), X at an odd base or row stride (K itself a
-// multiple of 8) in fewer than 128 workgroups (the same), more
-// than 128 MB of weights (the k loop then streams from HBM; of ten shapes
-// measured there this kernel was 6 and 9% faster on two and 5 to 33% slower on
-// the others), X beyond one launch's 32-bit offsets, and every call for which a knob or a schedule
-// record has chosen among those kernels.
+// The choice depends on the shape, X's alignment and whether C = A B or C += A B
+// is asked for, not on the result type, so a bf16 result stays the rounding of
+// the fp32 one.  Where a caller's scratch holds the plan without this kernel's
+// planes but not with them (below what llk_swiglu_scratch_size and
+// llk_describe_launch answer), that plan runs.  Kept on the other kernels:
+//  * 512 or fewer k, and X off the 16 bytes with K a multiple of 8 in fewer than
+//    128 64 x 64 tiles.  Not for speed: over 300 random shapes each the faster
+//    of both kernels is 1.74x and 1.72x the plan kept here.  The tests of those
+//    kernels' launches hold such shapes to them (test_gpu_code_object.py's wide
+//    tiles at K = 512 and padded X at 300 x 640 x 1000, test_tools_cpu.py's
+//    bucket and padded plans).
+//  * C += A B with 513..768 k, its partial planes being part of the scratch
+//    that its callers size: 1.75x over 300 shapes.
+//  * more than 128 MB of weights: the k loop then streams from HBM, and of 300
+//    shapes 2 are over 5% faster with the flex tile kernel (1.001x in all).
+//  * X beyond one launch's 32-bit offsets, and every call for which a knob or a
+//    schedule record has chosen among the other kernels.
 Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const llk_tensor2d* x,
                  size_t max_ws = SIZE_MAX, bool accumulate = false, bool out_bf16 = true,
                  bool rowmajor = false) {
   Plan p = plan_launch_large(nmat, M, K, KB, NB, x, max_ws, accumulate, out_bf16);
   p.need = p.ws_bytes;
   if (M <= 64 && llk::tunable("flex_tile") <= 1) {
-    // The decode tile kernel unsplit, narrower outputs (N <= 2176) and calls for
-    // which a knob or a schedule record has chosen keep their plans, which
-    // callers and tests hold this library to.
+    // Kept: the decode tile kernel unsplit (one launch already), calls for
+    // which a knob or a schedule record has chosen, and N <= 2176, where
+    // test_gpu_decode_tile.py and test_gpu_code_object.py hold the decode tile
+    // kernel's launches (over 300 random shapes there the choice would be 1.05x).
     llk::ScheduleEntry se;
     if (NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws ||
         llk::tunable("flex_tile") == 0 || llk::tunable("decode_max_m") != 64 || llk::tunable("decode_splits") > 0 ||
@@ -1023,9 +1032,9 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
         std::min(chain_steps(ref, nmat, M, KB), chain_steps(ref32, nmat, M, KB));
     // X rows that start inside a 128-byte line (whose lines are read twice)
     // slow a step by 8%, rows off the 16 bytes by 20% and at odd elements by
-    // 25% (K = 1600 against 1599 and 1598, N = 4288, M = 3779: 60.8, 67.1 and
-    // 67.4 us with the larger tiles, 18.2 to 20.1 us at M = 400).  Told from K,
-    // the stride of dense rows: a view's own stride must not change the sums.
+    // 25%; the models fit within 4% of their mean in each class with these.
+    // Told from K, the stride of dense rows: a view's own stride must not change
+    // the sums.
     const bool aligned = x_vec_ok(x);
     const double slow = aligned ? (K % 64 != 0 ? 1.08 : 1.0) : (K & 1 ? 1.25 : 1.20);
     double best = 0.97 * plan_us(ref, nmat, M, KB, NB);

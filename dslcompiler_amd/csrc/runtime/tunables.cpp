@@ -38,10 +38,10 @@ struct Knob {
 //                    take the wide tile kernel (16 B columns per matrix, B = 7
 //                    or 11) where its whole waves beat the 128-column tile;
 //                    0 = never; 7 or 11 = that width whenever it applies.
-// flex_tile:         1 = the cost model may take the flex tile kernel, and up
-//                    to 64 rows the small-M kernel unsplit in place of a k
-//                    split, as long as no other knob of the kernels compared
-//                    has been set; 0 = neither; 222, 224 or 244 = that tile (64 x
+// flex_tile:         1 = the cost model may take the flex tile kernel (above
+//                    64 rows, and below for K < 64), and up to 64 rows the
+//                    small-M kernel unsplit in place of a k split, as long as
+//                    no other knob of the kernels compared has been set; 0 = neither; 222, 224 or 244 = that tile (64 x
 //                    64, 64 x 128 or 128 x 128 MFMA rows), tile_splits its k
 //                    splits.
 // kernel_fn_rowmajor: 1 = the KernelFn entries read device weights with

@@ -355,9 +355,10 @@ int llk_fill_normal_bf16(uint64_t seed, uint64_t stream, float sigma,
  * of a partial last wave of tiles may run as a separate k-split launch;
  * 0: never; a forced "tile_splits" also turns it off), "tile_wide" (1:
  * the cost model may take the wide SwiGLU tiles; 0: never; 7 or 11: that
- * width), "flex_tile" (1: the cost model may take the flex tile kernel,
- * and up to 64 rows the small-M kernel unsplit in place of a k split; 0:
- * neither; 222, 224 or 244: that tile, with "tile_splits" as its k splits), "kernel_fn_rowmajor" (1: the KernelFn entries -- SwiGLU and, from
+ * width), "flex_tile" (1: the cost model may take the flex tile kernel --
+ * above 64 rows, and below for K < 64 -- and up to 64 rows the small-M kernel
+ * unsplit in place of a k split; 0: neither; 222, 224 or 244: that tile, with
+ * "tile_splits" as its k splits), "kernel_fn_rowmajor" (1: the KernelFn entries -- SwiGLU and, from
  * the object-code level, matmul -- read device weights
  * with aligned rows straight into the kernels' row-major forms; 0: they
  * pack the weights on every call), "max_workspaces" (library-owned
