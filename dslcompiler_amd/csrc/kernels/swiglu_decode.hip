@@ -443,7 +443,8 @@ static int skinny_threads_w(int W) {
 // same columns, so the epilogue is register-local; GEMM: column groups c and
 // 2 + c).  With S > 1 workgroup (columns, s) covers the 64-k blocks
 // [s kbs, (s + 1) kbs) and writes fp32 partials in the layout of
-// skinny_kernel's, which skinny_reduce_kernel adds in split order.
+// skinny_kernel's, which skinny_reduce_kernel adds in split order.  (Row-major,
+// 64 rows: a workgroup may hold several parts of k, see plane_kb.)
 //
 // MT (32-row MFMA tiles per wave: 1, 2, 4) sets the rows a workgroup holds,
 // 64 MT: MT = 1 for M <= 64 (decode), 2 and 4 for mid M (65..256 rows, one
@@ -466,6 +467,7 @@ struct DecTileArgs {
   float* part;        // [S][NMAT][rows][n_pad] fp32 partials (S > 1)
   int64_t ldx, ldy;
   int M, N, KB, NB, S, kbs, n_pad, rows;
+  int plane_kb;  // 64-k steps of a part sum: kbs, or (RM, 64 rows) a part of it
   bool accumulate;  // GEMM only, S == 1: y += x w (the existing y read in its type)
   // The row-major form (RM): w0 / w1 are bf16 [K, N] with rows of ldw0 /
   // ldw1 elements instead of packed payloads.
@@ -614,8 +616,39 @@ __global__ __launch_bounds__(256) void decode_tile_kernel(DecTileArgs a) {
   const int xm = mh * 32 * MT + (lane & 31);                  // the B operand's row (t = 0)
   const uint8_t* const b_rd = smem + kDecW + xm * 128;        // + t * 4 KiB: tile t's rows
   int slot = 0, fill = kAhead;
+  // The plane of the part that ends at step kb of this workgroup: one for all
+  // of the first workgroup's along k, then one for each.
+  auto plane_of = [&](int kb) {
+    return RM && MT == 1 ? (kb0 == 0 ? 0 : (kb0 + kb - 1) / a.plane_kb - a.kbs / a.plane_kb + 1)
+                         : split;
+  };
+  // Stores acc as the partial plane `plane` (the reduce reads rows < M only).
+  const int n_col = NMAT == 2 ? grp * 64 + cg * 32 : nb * kPackN + cg * 32;
+  auto store_plane = [&](int plane, int m, int t) {
+    if (m >= a.M) return;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int mat = NMAT == 2 ? p : 0;
+        const int n = n_col + (NMAT == 2 ? 0 : p * 64) + 8 * g + 4 * (lane >> 5);
+        float* dst = a.part + (((size_t)plane * NMAT + mat) * a.rows + m) * a.n_pad + n;
+        *reinterpret_cast<f32x4*>(dst) = f32x4{acc[p][t][4 * g], acc[p][t][4 * g + 1],
+                                               acc[p][t][4 * g + 2], acc[p][t][4 * g + 3]};
+      }
+  };
   if constexpr (MT == 1) {
-    for (int kb = 0; kb < nkb; ++kb) {
+    // A row-major workgroup may hold several parts of k (a.plane_kb steps each),
+    // one after the other, the ring running on: the first along k adds them up
+    // in order, as the reduce would, the others store a plane for each.
+    f32x16 total[2];
+    if constexpr (RM)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) total[p][r] = 0.0f;
+    int end = RM ? min(nkb, a.plane_kb) : nkb;
+    for (int kb = 0;;) {
       wait_vmcnt<kLoads * (kAhead - 1)>();  // this wave's loads of step kb have landed
       __syncthreads();                      // ... every wave's; slot `fill` (step kb - 1) is free
       issue(kb + kAhead, fill);
@@ -635,7 +668,24 @@ __global__ __launch_bounds__(256) void decode_tile_kernel(DecTileArgs a) {
 #pragma unroll
         for (int p = 0; p < 2; ++p) acc[p][0] = mfma32(A[p][kq], Bx[kq], acc[p][0]);
       slot = slot + 1 == kDecSlots ? 0 : slot + 1;
+      if (++kb != end) continue;
+      if (!RM || kb == nkb) break;
+      if (kb0 != 0) store_plane(plane_of(kb), xm, 0);
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          total[p][r] += acc[p][0][r];
+          acc[p][0][r] = 0.0f;
+        }
+      end = min(nkb, end + a.plane_kb);
     }
+    if constexpr (RM)
+      if (kb0 == 0 && a.plane_kb < a.kbs)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[p][0][r] = total[p][r] + acc[p][0][r];
   } else {
     // 2 MT MFMAs per 16-k quarter kq, and the LDS serves 4 (2 + MT) KiB of
     // operands per quarter to the workgroup's waves beside the ring's DMA
@@ -691,26 +741,18 @@ __global__ __launch_bounds__(256) void decode_tile_kernel(DecTileArgs a) {
 
   // acc[p][t] register r, lane l: row m = 32 (MT h + t) + l % 32, column
   // 8 (r / 4) + 4 (l / 32) + r % 4 of the wave's 32-column group of operand p.
-  const int n_col = NMAT == 2 ? grp * 64 + cg * 32 : nb * kPackN + cg * 32;
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int m = xm + 32 * t;
     if (MT > 1 && m >= a.rows) continue;  // rows past M's last 32-row group
+    if (a.S > 1) {
+      store_plane(plane_of(nkb), m, t);
+      continue;
+    }
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int n_off = 8 * g + 4 * (lane >> 5);
-      if (a.S > 1) {
-        if (m < a.M) {  // the reduce reads rows < M only
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const int mat = NMAT == 2 ? p : 0;
-            const int n = n_col + (NMAT == 2 ? 0 : p * 64) + n_off;
-            float* dst = a.part + (((size_t)split * NMAT + mat) * a.rows + m) * a.n_pad + n;
-            *reinterpret_cast<f32x4*>(dst) = f32x4{acc[p][t][4 * g], acc[p][t][4 * g + 1],
-                                                   acc[p][t][4 * g + 2], acc[p][t][4 * g + 3]};
-          }
-        }
-      } else if constexpr (NMAT == 2) {
+      if constexpr (NMAT == 2) {
         float v[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -749,7 +791,8 @@ static hipError_t launch_decode_tile_t(const DecTileArgs& a, const llk::ModuleFn
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), kLds, lds_set);
     if (e != hipSuccess) return e;
   }
-  const unsigned groups = (unsigned)((NMAT == 2 ? a.NB * 2 : a.NB) * a.S);
+  const int wg_splits = (a.KB + a.kbs - 1) / a.kbs;
+  const unsigned groups = (unsigned)((NMAT == 2 ? a.NB * 2 : a.NB) * wg_splits);
   hipError_t e = launch_kernel(mod, reinterpret_cast<const void*>(fn),
                                &decode_tile_symbol<NMAT, OUT, MT, RM>, dim3(groups), dim3(256), kLds,
                                s, a);
@@ -899,6 +942,7 @@ hipError_t llk_launch_decode_tile(int mode, const uint16_t* x, int64_t ldx, cons
   a.NB = NB;
   a.S = S < 1 ? 1 : S;
   a.kbs = (KB + a.S - 1) / a.S;
+  a.plane_kb = a.kbs;
   a.n_pad = NB * kPackN;
   a.rows = skinny_rows(M);
   a.accumulate = accumulate;
@@ -924,11 +968,14 @@ hipError_t llk_launch_decode_tile(int mode, const uint16_t* x, int64_t ldx, cons
 // payload): w0 / w1 are bf16 [K, N] with rows of ldw0 / ldw1 elements,
 // llk_decode_rowmajor_fits must hold for each; otherwise as
 // llk_launch_decode_tile (grid, k splits, workspace and results: the same
-// MFMA operands in the same order, so the same bits as the packed form).
+// MFMA operands in the same order, so the same bits as the packed form).  Up to
+// 64 rows the S parts of k may lie in wg_splits workgroups along k (0: S of
+// them), ceil(S / wg_splits) in each; ws then holds S planes less those that
+// the first of them adds up itself (none for one workgroup).
 hipError_t llk_launch_decode_rowmajor(int mode, const uint16_t* x, int64_t ldx,
                                       const uint16_t* w0, int64_t ldw0, const uint16_t* w1,
                                       int64_t ldw1, void* y, int64_t ldy, int M, int N, int K,
-                                      int S, void* ws, int out, bool accumulate,
+                                      int S, int wg_splits, void* ws, int out, bool accumulate,
                                       const llk::ModuleFns* mod, hipStream_t s) {
   using namespace llk_gfx950;
   if (N < 1 || !llk_decode_rowmajor_fits(M, K, ldx, w0, ldw0, N) ||
@@ -950,11 +997,16 @@ hipError_t llk_launch_decode_rowmajor(int mode, const uint16_t* x, int64_t ldx,
   a.KB = K / 64;
   a.NB = (N + kPackN - 1) / kPackN;
   a.S = S < 1 ? 1 : S;
-  a.kbs = (a.KB + a.S - 1) / a.S;
+  const int parts = a.S;
+  a.plane_kb = (a.KB + parts - 1) / parts;
+  const int per = wg_splits < 1 || dec_mt(M) > 1 ? 1 : (parts + wg_splits - 1) / wg_splits;
+  a.kbs = a.plane_kb * per;  // of each workgroup
+  a.S = a.kbs >= a.KB ? 1 : 1 + parts - per;
   a.n_pad = a.NB * kPackN;
   a.rows = skinny_rows(M);
   a.accumulate = accumulate;
-  if (a.S > 1 && (ws == nullptr || (int64_t)(a.S - 1) * a.kbs >= a.KB)) return hipErrorInvalidValue;
+  if ((int64_t)(parts - 1) * a.plane_kb >= a.KB || (a.S > 1 && ws == nullptr))
+    return hipErrorInvalidValue;
   const int mt = dec_mt(M);
 #if !defined(LLK_CO_OP) || LLK_CO_OP == 1
   if (mode == 1) {

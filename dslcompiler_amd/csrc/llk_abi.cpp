@@ -60,7 +60,7 @@ bool llk_decode_rowmajor_fits(int M, int64_t K, int64_t ldx, const void* w, int6
 hipError_t llk_launch_decode_rowmajor(int mode, const uint16_t* x, int64_t ldx,
                                       const uint16_t* w0, int64_t ldw0, const uint16_t* w1,
                                       int64_t ldw1, void* y, int64_t ldy, int M, int N, int K,
-                                      int S, void* ws, int out, bool accumulate,
+                                      int S, int wg_splits, void* ws, int out, bool accumulate,
                                       const llk::ModuleFns* mod, hipStream_t s);
 bool llk_tile_rowmajor_fits(int M, int64_t K, int64_t ldx, const void* w, int64_t ldw, int64_t N);
 hipError_t llk_launch_tile_rowmajor(int mode, const uint16_t* x, int64_t ldx, const uint16_t* w0,
@@ -372,6 +372,7 @@ struct Plan {
   bool too_large = false;  // tile path: K beyond the kernel's 32-bit offsets
   int64_t head_nb = 0;   // tile path: leading n-blocks launched unsplit (S applies to the rest)
   int flex = 0;          // flex tile kernel: its tile (222, 224, 244); S as above
+  int wg_splits = 0;     // row-major decode tile kernel: workgroups along k (0: S)
   size_t need = 0;       // workspace the launches use; ws_bytes: what a caller's scratch holds
   int wide = 0;          // tile path, fused SwiGLU with bf16 output: the wide kernel's B
                          // (16 B columns per tile and matrix; 0 = the 128-column kernel)
@@ -992,14 +993,32 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     if (!rowmajor) return q;
     // Row-major weights have no small-M form (those the decode tile kernel
     // cannot read are packed, and take q): the decode tile kernel with that
-    // kernel's k parts as its splits.  Both run the same MFMAs over each part
-    // and add the parts in order, so the result is the packed call's bit for
-    // bit.  It costs a synchronous KernelFn call 14% in the mean of 36 shapes
-    // (M = 7, K = 1728, N = 3456 23.7 -> 26.3 us in 7 splits for 4).
+    // kernel's k parts.  Both run the same MFMAs over each part and add the
+    // parts in order, so the result is the packed call's bit for bit.  A
+    // workgroup holds one or more parts, as many as the fastest of a model: the
+    // steps of the rounds, and with several workgroups along k the reduce and
+    // its planes (150 measured SwiGLU shapes, M 1..64, K 512..5120, N 2184..14336:
+    // a synchronous KernelFn call takes 5% longer in the geometric mean than at
+    // the decode tile kernel's own split count, always the fastest 4.6%, one
+    // part to each workgroup 14%; M = 9, K = 2688, N = 8032 37.6 us at its own
+    // two splits, 47.1 with a workgroup for each of the seven parts).
     if (p.dtile && q.skinny && !q.dtile) {
-      const int64_t part = chain_steps(q, nmat, M, KB);
-      p.S = (int)((KB + part - 1) / part);
-      p.ws_bytes = p.need = llk_skinny_workspace_bytes(nmat, (int)M, (int)(NB * 128), p.S);
+      const int64_t part = chain_steps(q, nmat, M, KB), parts = (KB + part - 1) / part;
+      double best = 0.0;
+      for (int64_t w = 1; w <= parts; ++w) {
+        const int64_t per = (parts + w - 1) / w, along = (parts + per - 1) / per;
+        const int64_t wgs = along * (nmat == 2 ? NB * 2 : NB);
+        const int planes = along == 1 ? 1 : (int)(1 + parts - per);
+        const double step = wgs <= 256 ? 0.31 : wgs <= 512 ? 0.64 : 0.54 * (double)wgs / 256.0;
+        const double us = step * (double)std::min(per * part, KB) +
+                          (planes > 1 ? 1.0 + 0.53 * planes * nmat * M * NB * 512e-6 : 0.0);
+        if (w > 1 && us >= best) continue;
+        best = us;
+        p.wg_splits = (int)w;
+        p.ws_bytes = p.need =
+            llk_skinny_workspace_bytes(nmat, (int)M, (int)(NB * 128), planes);
+      }
+      p.S = (int)parts;
     }
     return p;
   }
@@ -1983,8 +2002,7 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
   } else {
     e = llk_launch_decode_rowmajor(mode, xd, x->stride0, wgd, wg->stride0, wud,
                                    mode == 1 ? wu->stride0 : 0, y->data, y->stride0, (int)M, (int)N,
-                                   (int)K, S, ws, out_dtype, accumulate,
-                                   mod, s);
+                                   (int)K, S, p.wg_splits, ws, out_dtype, accumulate, mod, s);
   }
   release_workspace(dev, held, s);
   return e == hipSuccess ? LLK_OK

@@ -292,11 +292,16 @@ def test_kernel_fn_rowmajor_matches_packed(llk, gpu, orc, M, K, N, ldw):
     assert_parity_bf16(got, orc.swiglu(x, wg, wu)[0], f"KernelFn row-major M={M}")
 
 
-# One shape per small-M form that the packed path takes in place of a k split
-# (N > 2176): operation, rows above 32 or not, 32-column groups per workgroup.
+# Shapes where the packed path takes the small-M kernel in place of a k split (N
+# > 2176): operation, M, K, N and its 32-column groups per workgroup, one for
+# each of its forms (rows above 32 or not); then, in the KernelFn, several parts
+# of k in each of several workgroups along k (the last with fewer parts, or a
+# shorter part) and one part in each.
 ONE_LAUNCH = [(0, 26, 576, 2184, 1), (0, 11, 1728, 8200, 2), (0, 54, 704, 2184, 1),
               (0, 1, 640, 2304, 1), (3, 17, 512, 2184, 1), (3, 27, 1152, 2184, 2),
-              (3, 37, 576, 2208, 1), (3, 42, 896, 8200, 2)]
+              (3, 37, 576, 2208, 1), (3, 42, 896, 8200, 2),
+              (0, 9, 1216, 2392, 1), (0, 24, 1408, 2240, 1), (0, 17, 1088, 2184, 1),
+              (3, 6, 1600, 2488, 2), (3, 21, 832, 2256, 1)]
 
 
 @pytest.mark.parametrize("op,M,K,N,W", ONE_LAUNCH)
