@@ -767,7 +767,8 @@ Plan plan_launch_large(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
 // it, by up to 26%: C = A B 3501 x 640 x 12384 70.5 us without it, 95.7 with,
 // SwiGLU 74 x 896 x 11104 12.5 and 15.7 us.)  Over them the choice runs 1.165x
 // the plan without this kernel in the geometric mean, the fastest measured
-// 1.171x; where it differs (2527) 1.35x, at 26 over 3% slower.
+// 1.172x; where it differs (2632) 1.34x, at 56 over 3% slower.  On weights that
+// stay in the 256 MB cache (3000 of the shapes): 1.179x, at 23 slower.
 //   us = base + slow kbs step[n] + out (MB of Y, or of planes when S > 1)
 //          + weights (MB of weights)
 // with n = ceil(workgroups / 256) and kbs = 64-k steps per split: the
@@ -1056,7 +1057,10 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     // the sums.
     const bool aligned = x_vec_ok(x);
     const double slow = aligned ? (K % 64 != 0 ? 1.08 : 1.0) : (K & 1 ? 1.25 : 1.20);
-    double best = 0.97 * plan_us(ref, nmat, M, KB, NB);
+    // Taken when modelled 1% faster.  With its weights in cache this kernel gains
+    // up to 10% on the decode tile kernel, which streams them past the caches,
+    // so a wider margin would lose there what it saves on weights from HBM.
+    double best = 0.99 * plan_us(ref, nmat, M, KB, NB);
     if (!aligned && K % 8 == 0 && (M + 63) / 64 * (NB * 2 * nmat) < 128) return p;
     const double y_mb = M * NB * 128 * 3e-6, w_mb = KB * NB * 16384e-6 * nmat;
     for (const FlexModel& f : kFlex) {
