@@ -269,7 +269,7 @@ int get_workspace(int dev, size_t need, size_t asked, llk_kernel_context* ctx, v
   std::lock_guard<std::mutex> lk(st.mu);
   Workspace* w = nullptr;
   if (st.ws.find(key) == st.ws.end()) {
-    const size_t cap = (size_t)std::max<int64_t>(1, llk::tunable("max_workspaces"));
+    const size_t cap = (size_t)std::max<int64_t>(1, llk::tunable(llk::Knob::max_workspaces));
     while (st.ws.size() >= cap && evict_one_workspace(st, nullptr)) {
     }
   }
@@ -391,11 +391,11 @@ struct SplitCost {
 };
 
 SplitCost best_split(int nmat, int64_t rows, int64_t KB, int64_t NB, int64_t forced) {
-  const int64_t min_kb = std::max<int64_t>(1, llk::tunable("tile_min_kb"));
+  const int64_t min_kb = std::max<int64_t>(1, llk::tunable(llk::Knob::tile_min_kb));
   int64_t smax = std::min<int64_t>(64, std::max<int64_t>(1, KB / min_kb));
   if (forced > 0) smax = std::min(forced, KB);
   const int64_t tiles = (rows + 255) / 256 * (nmat == 2 ? NB : (NB + 1) / 2);
-  const int64_t per_wave = std::max<int64_t>(1, llk::tunable("tile_wgs_per_wave"));
+  const int64_t per_wave = std::max<int64_t>(1, llk::tunable(llk::Knob::tile_wgs_per_wave));
   SplitCost best{1, 0.0};
   for (int64_t S = forced > 0 ? smax : 1; S <= smax; ++S) {
     const int64_t kbs = (KB + S - 1) / S;
@@ -423,17 +423,17 @@ struct TilePlan {
 };
 
 TilePlan tile_plan(int nmat, int64_t rows, int64_t KB, int64_t NB, int64_t db_splits) {
-  int64_t forced = llk::tunable("tile_splits");
+  int64_t forced = llk::tunable(llk::Knob::tile_splits);
   if (forced <= 0) forced = db_splits;
   const SplitCost all = best_split(nmat, rows, KB, NB, forced);
   if (forced > 0) return {all.S, 0, all.cost};
   const int64_t nb_per_tile = nmat == 2 ? 1 : 2;
   const int64_t tm = (rows + 255) / 256, tn = (NB + nb_per_tile - 1) / nb_per_tile;
-  const int64_t per_wave = std::max<int64_t>(1, llk::tunable("tile_wgs_per_wave"));
+  const int64_t per_wave = std::max<int64_t>(1, llk::tunable(llk::Knob::tile_wgs_per_wave));
   const int64_t head_tn = tm * tn / per_wave * per_wave / tm;  // columns of q whole waves
   TilePlan best{all.S, 0, all.cost};
   double best_cost = all.cost;
-  if (llk::tunable("tile_tail_split") != 0 && head_tn > 0 && head_tn < tn) {
+  if (llk::tunable(llk::Knob::tile_tail_split) != 0 && head_tn > 0 && head_tn < tn) {
     const int64_t head_nb = head_tn * nb_per_tile;
     const double head = (double)((tm * head_tn + per_wave - 1) / per_wave) * (double)(KB + 2);
     const SplitCost tail = best_split(nmat, rows, KB, NB - head_nb, 0);
@@ -461,10 +461,10 @@ struct WideChoice {
 };
 
 WideChoice wide_choice(int64_t rows, int64_t N, int64_t KB, double std_cost, int64_t forced_s) {
-  const int64_t knob = llk::tunable("tile_wide");
+  const int64_t knob = llk::tunable(llk::Knob::tile_wide);
   if (knob == 0) return {};
-  const int64_t per_wave = std::max<int64_t>(1, llk::tunable("tile_wgs_per_wave"));
-  const int64_t min_kb = std::max<int64_t>(1, llk::tunable("tile_min_kb"));
+  const int64_t per_wave = std::max<int64_t>(1, llk::tunable(llk::Knob::tile_wgs_per_wave));
+  const int64_t min_kb = std::max<int64_t>(1, llk::tunable(llk::Knob::tile_min_kb));
   const int64_t tm = (rows + 255) / 256;
   WideChoice best;
   double best_cost = 0.97 * std_cost;
@@ -547,8 +547,8 @@ struct SmallMChoice {
 
 SmallMChoice small_m_choice(int nmat, int64_t M, int64_t KB, int64_t NB, int64_t force_w,
                             int64_t force_s) {
-  const int64_t target = std::max<int64_t>(1, llk::tunable("decode_target_wgs"));
-  const int64_t min_kb = std::max<int64_t>(1, llk::tunable("decode_min_kb"));
+  const int64_t target = std::max<int64_t>(1, llk::tunable(llk::Knob::decode_target_wgs));
+  const int64_t min_kb = std::max<int64_t>(1, llk::tunable(llk::Knob::decode_min_kb));
   const int64_t rows = (M + 31) / 32 * 32;
   auto cost = [&](int64_t W, int64_t S, int64_t* s_out) {
     const int64_t kbs = (KB + S - 1) / S;
@@ -595,8 +595,8 @@ SmallMChoice small_m_choice(int nmat, int64_t M, int64_t KB, int64_t NB, int64_t
 // step: 64 columns of both SwiGLU matrices, 128 of the GEMM's).  A forced
 // split count (> 0) is kept.
 int decode_tile_splits(int nmat, int64_t M, int64_t KB, int64_t NB, int64_t force_s) {
-  const int64_t target = std::max<int64_t>(1, llk::tunable("decode_target_wgs"));
-  const int64_t min_kb = std::max<int64_t>(1, llk::tunable("decode_min_kb"));
+  const int64_t target = std::max<int64_t>(1, llk::tunable(llk::Knob::decode_target_wgs));
+  const int64_t min_kb = std::max<int64_t>(1, llk::tunable(llk::Knob::decode_min_kb));
   const int64_t rows = (M + 31) / 32 * 32;
   const int64_t groups = nmat == 2 ? NB * 2 : NB;
   int64_t s_lo = 1, s_hi = std::min<int64_t>(64, std::max<int64_t>(1, KB / min_kb));
@@ -632,11 +632,11 @@ Plan plan_launch_base(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
   Plan p;
   llk::ScheduleEntry se;
   const bool have_db = db_entry(nmat, M, &se);
-  if (M <= std::min<int64_t>(64, llk::tunable("decode_max_m"))) {
+  if (M <= std::min<int64_t>(64, llk::tunable(llk::Knob::decode_max_m))) {
     p.skinny = true;
-    int64_t gw = llk::tunable("decode_group_width");
+    int64_t gw = llk::tunable(llk::Knob::decode_group_width);
     if (gw <= 0 && have_db && (se.BN == 32 || se.BN == 64 || se.BN == 128)) gw = se.BN / 32;
-    int64_t S = llk::tunable("decode_splits");
+    int64_t S = llk::tunable(llk::Knob::decode_splits);
     if (S <= 0 && have_db && se.grain_size > 0) S = se.grain_size;
     auto fit_splits = [&](int s) {
       size_t ws = llk_skinny_workspace_bytes(nmat, (int)M, (int)(NB * 128), s);
@@ -649,7 +649,7 @@ Plan plan_launch_base(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
     // The decode tile kernel unless a width is forced (the small-M kernel's
     // own knob, or its schedule record) or the shape does not fit it; when
     // X is unknown (sizing), the larger of the two workspaces.
-    if (llk::tunable("decode_tile") != 0 && gw <= 0 &&
+    if (llk::tunable(llk::Knob::decode_tile) != 0 && gw <= 0 &&
         llk_decode_tile_fits((int)M, K, x ? x->stride0 : K)) {
       const auto d = fit_splits(decode_tile_splits(nmat, M, KB, NB, S));
       if (!x) {
@@ -680,9 +680,9 @@ Plan plan_launch_base(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
   // The wide kernel: fused SwiGLU, bf16 output.  A forced split count or a
   // DB entry with one keeps the 128-column kernel unless tile_wide forces a
   // width (which then takes the forced split count).
-  const int64_t forced_s = llk::tunable("tile_splits");
+  const int64_t forced_s = llk::tunable(llk::Knob::tile_splits);
   const bool split_forced = forced_s > 0 || (have_db && se.grain_size > 1);
-  const bool wide_forced = llk::tunable("tile_wide") == 7 || llk::tunable("tile_wide") == 11;
+  const bool wide_forced = llk::tunable(llk::Knob::tile_wide) == 7 || llk::tunable(llk::Knob::tile_wide) == 11;
   if (nmat == 2 && out_bf16 && !accumulate && (!split_forced || wide_forced)) {
     const WideChoice wc = wide_choice(rows, NB * 128, KB, tp.cost, forced_s);
     if (wc.B) {
@@ -733,9 +733,9 @@ Plan plan_launch_base(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
 // larger of the two workspaces.
 Plan plan_launch_large(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB,
                        const llk_tensor2d* x, size_t max_ws, bool accumulate, bool out_bf16) {
-  if (M > 64 && M <= std::min<int64_t>(256, llk::tunable("midm_max_m")) &&
-      llk::tunable("decode_tile") != 0 && llk_decode_tile_fits((int)M, K, x ? x->stride0 : K)) {
-    int64_t forced = llk::tunable("decode_splits");
+  if (M > 64 && M <= std::min<int64_t>(256, llk::tunable(llk::Knob::midm_max_m)) &&
+      llk::tunable(llk::Knob::decode_tile) != 0 && llk_decode_tile_fits((int)M, K, x ? x->stride0 : K)) {
+    int64_t forced = llk::tunable(llk::Knob::decode_splits);
     llk::ScheduleEntry se;
     if (forced <= 0 && db_entry(nmat, M, &se) && se.grain_size > 0) forced = se.grain_size;
     int s = decode_tile_splits(nmat, M, KB, NB, forced);
@@ -975,16 +975,16 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
                  bool rowmajor = false) {
   Plan p = plan_launch_large(nmat, M, K, KB, NB, x, max_ws, accumulate, out_bf16);
   p.need = p.ws_bytes;
-  if (M <= 64 && llk::tunable("flex_tile") <= 1) {
+  if (M <= 64 && llk::tunable(llk::Knob::flex_tile) <= 1) {
     // Kept: the decode tile kernel unsplit (one launch already), calls for
     // which a knob or a schedule record has chosen, and N <= 2176, where
     // test_gpu_decode_tile.py and test_gpu_code_object.py hold the decode tile
     // kernel's launches (over 300 random shapes there the choice would be 1.05x).
     llk::ScheduleEntry se;
     if (NB < 18 || (p.dtile && p.S == 1) || p.ws_bytes > max_ws ||
-        llk::tunable("flex_tile") == 0 || llk::tunable("decode_max_m") != 64 || llk::tunable("decode_splits") > 0 ||
-        llk::tunable("decode_group_width") > 0 || llk::tunable("decode_tile") != 1 ||
-        llk::tunable("decode_target_wgs") != 256 || llk::tunable("decode_min_kb") != 2 ||
+        llk::tunable(llk::Knob::flex_tile) == 0 || llk::tunable(llk::Knob::decode_max_m) != 64 || llk::tunable(llk::Knob::decode_splits) > 0 ||
+        llk::tunable(llk::Knob::decode_group_width) > 0 || llk::tunable(llk::Knob::decode_tile) != 1 ||
+        llk::tunable(llk::Knob::decode_target_wgs) != 256 || llk::tunable(llk::Knob::decode_min_kb) != 2 ||
         (db_entry(nmat, M, &se) && (se.grain_size > 0 || se.BN == 32 || se.BN == 64 || se.BN == 128)))
       return p;
     const Plan ref = max_ws != SIZE_MAX
@@ -1023,8 +1023,8 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     }
     return p;
   }
-  const int64_t knob = llk::tunable("flex_tile");
-  const int64_t forced_s = llk::tunable("tile_splits");
+  const int64_t knob = llk::tunable(llk::Knob::flex_tile);
+  const int64_t forced_s = llk::tunable(llk::Knob::tile_splits);
   int cfg = 0;
   int64_t S = 1;
   if (knob > 1) {
@@ -1034,10 +1034,10 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
   } else {
     if (knob == 0 || M <= 64 || KB <= (accumulate ? 12 : 8) ||
         KB * NB * nmat > 8192 || (p.chunk > 0 && p.chunk < M) || p.too_large ||
-        p.ws_bytes > max_ws || forced_s > 0 || llk::tunable("tile_wide") != 1 || llk::tunable("tile_wgs_per_wave") != 256 ||
-        llk::tunable("tile_tail_split") != 1 || llk::tunable("tile_min_kb") != 4 ||
-        llk::tunable("midm_max_m") != 128 || llk::tunable("decode_tile") != 1 ||
-        llk::tunable("decode_splits") > 0)
+        p.ws_bytes > max_ws || forced_s > 0 || llk::tunable(llk::Knob::tile_wide) != 1 || llk::tunable(llk::Knob::tile_wgs_per_wave) != 256 ||
+        llk::tunable(llk::Knob::tile_tail_split) != 1 || llk::tunable(llk::Knob::tile_min_kb) != 4 ||
+        llk::tunable(llk::Knob::midm_max_m) != 128 || llk::tunable(llk::Knob::decode_tile) != 1 ||
+        llk::tunable(llk::Knob::decode_splits) > 0)
       return p;
     llk::ScheduleEntry se;
     if (db_entry(nmat, M, &se) && se.grain_size > 0) return p;
@@ -1925,7 +1925,7 @@ int rowmajor_with_module(int mode, const llk_tensor2d* x, const llk_tensor2d* wg
                          llk_kernel_context* ctx, const ModuleFns* mod, bool accumulate,
                          bool* taken) {
   *taken = false;
-  if (llk::tunable("kernel_fn_rowmajor") == 0) return LLK_OK;
+  if (llk::tunable(llk::Knob::kernel_fn_rowmajor) == 0) return LLK_OK;
   const int64_t M = x->dim0, K = x->dim1, N = wg->dim1;
   if (M < 1 || N < 1 || K < 1 || y->dim0 != M || y->dim1 != N || !x_vec_ok(x)) return LLK_OK;
   if (wg->stride1 != 1 || (mode == 1 && (!wu || wu->stride1 != 1 || wu->dim1 != N))) return LLK_OK;

@@ -1,16 +1,9 @@
 // tunables.cpp -- storage for the knobs declared in tunables.h.
 #include "tunables.h"
 
-#include <atomic>
 #include <cstring>
 
 namespace llk {
-namespace {
-
-struct Knob {
-  const char* name;
-  std::atomic<int64_t> value;
-};
 
 // decode_max_m:      largest M (<= 64) routed to the small-M bandwidth kernel.
 // decode_splits:     force its cross-workgroup k-split count (0 = cost model).
@@ -53,48 +46,38 @@ struct Knob {
 //                    stream, or per thread on the per-thread default
 //                    stream); beyond it the least recently used idle one is
 //                    freed once its last call has finished.
-Knob g_knobs[] = {
-    {"decode_max_m", {64}},
-    {"decode_splits", {0}},
-    {"decode_target_wgs", {256}},
-    {"decode_min_kb", {2}},
-    {"decode_group_width", {0}},
-    {"decode_tile", {1}},
-    {"midm_max_m", {128}},
-    {"tile_splits", {0}},
-    {"tile_wgs_per_wave", {256}},
-    {"tile_min_kb", {4}},
-    {"tile_tail_split", {1}},
-    {"tile_wide", {1}},
-    {"flex_tile", {1}},
-    {"kernel_fn_rowmajor", {1}},
-    {"max_workspaces", {16}},
+std::atomic<int64_t> g_knob_values[] = {
+#define LLK_KNOB(name, value) {value},
+    LLK_KNOBS(LLK_KNOB)
+#undef LLK_KNOB
 };
+
+namespace {
+
+constexpr const char* kNames[] = {
+#define LLK_KNOB(name, value) #name,
+    LLK_KNOBS(LLK_KNOB)
+#undef LLK_KNOB
+};
+
+std::atomic<int64_t>* find(const char* name) {
+  for (size_t i = 0; i < sizeof(kNames) / sizeof(*kNames); ++i)
+    if (std::strcmp(kNames[i], name) == 0) return &g_knob_values[i];
+  return nullptr;
+}
 
 }  // namespace
 
-int64_t tunable(const char* name) {
-  for (auto& k : g_knobs)
-    if (std::strcmp(k.name, name) == 0) return k.value.load(std::memory_order_relaxed);
-  return 0;
-}
-
 bool setTunable(const char* name, int64_t value) {
-  for (auto& k : g_knobs)
-    if (std::strcmp(k.name, name) == 0) {
-      k.value.store(value, std::memory_order_relaxed);
-      return true;
-    }
-  return false;
+  std::atomic<int64_t>* const v = find(name);
+  if (v) v->store(value, std::memory_order_relaxed);
+  return v != nullptr;
 }
 
 bool getTunable(const char* name, int64_t* value) {
-  for (auto& k : g_knobs)
-    if (std::strcmp(k.name, name) == 0) {
-      *value = k.value.load(std::memory_order_relaxed);
-      return true;
-    }
-  return false;
+  std::atomic<int64_t>* const v = find(name);
+  if (v) *value = v->load(std::memory_order_relaxed);
+  return v != nullptr;
 }
 
 }  // namespace llk
