@@ -285,10 +285,22 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(SkinnyArgs a, int ro
   f32x4 s[NMAT];
 #pragma unroll
   for (int p = 0; p < NMAT; ++p) s[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int sp = 0; sp < a.S; ++sp)
+  // Four planes in flight at a time, added in order: one after the other their
+  // latencies add up.
+  for (int sp = 0; sp < a.S; sp += 4) {
+    f32x4 v[4][NMAT];
 #pragma unroll
-    for (int p = 0; p < NMAT; ++p)
-      s[p] += *reinterpret_cast<const f32x4*>(a.part + (((size_t)sp * NMAT + p) * rows + m) * a.n_pad + n);
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int p = 0; p < NMAT; ++p)
+        v[u][p] = *reinterpret_cast<const f32x4*>(
+            a.part + (((size_t)min(sp + u, a.S - 1) * NMAT + p) * rows + m) * a.n_pad + n);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int p = 0; p < NMAT; ++p)
+        if (sp + u < a.S) s[p] += v[u][p];
+  }
   float v[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {

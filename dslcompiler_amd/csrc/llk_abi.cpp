@@ -998,11 +998,11 @@ Plan plan_launch(int nmat, int64_t M, int64_t K, int64_t KB, int64_t NB, const l
     // parts in order, so the result is the packed call's bit for bit.  A
     // workgroup holds one or more parts, as many as the fastest of a model: the
     // steps of the rounds, and with several workgroups along k the reduce and
-    // its planes (150 measured SwiGLU shapes, M 1..64, K 512..5120, N 2184..14336:
-    // a synchronous KernelFn call takes 5% longer in the geometric mean than at
-    // the decode tile kernel's own split count, always the fastest 4.6%, one
-    // part to each workgroup 14%; M = 9, K = 2688, N = 8032 37.6 us at its own
-    // two splits, 47.1 with a workgroup for each of the seven parts).
+    // its planes (fitted on 150 SwiGLU shapes, M 1..64, K 512..5120, N 2184..14336).
+    // Over 36 others a synchronous KernelFn call takes 2.6% longer in the
+    // geometric mean than at the decode tile kernel's own split count, 14% with a
+    // workgroup for each part (M = 9, K = 2688, N = 8032: 37.3 us at its own two
+    // splits, 38.7, and 47.1 with seven).
     if (p.dtile && q.skinny && !q.dtile) {
       const int64_t part = chain_steps(q, nmat, M, KB), parts = (KB + part - 1) / part;
       double best = 0.0;
