@@ -200,7 +200,8 @@ size_t llk_swiglu_scratch_size(int64_t M, int64_t N, int64_t K);
  * the reference's ShapeSpecialization + ScheduleSelection passes
  * (ShapeSpecialization.cpp:38-48, ScheduleSelection.cpp:46-67) for this
  * backend.  flags: LLK_PLAN_X_ALIGNED -- X rows are 16-byte aligned with
- * K % 8 == 0 (else the worst case, a padded copy of X, is assumed);
+ * K % 8 == 0 (else rows at any element, which the tile kernels copy to
+ * padded ones first);
  * LLK_PLAN_ACCUMULATE -- the plan of llk_gemm_bf16_accumulate (matmul only),
  * which always ends with the reduce launch that adds C and needs its
  * partial planes even unsplit; LLK_PLAN_OUT_F32 -- fused SwiGLU with an fp32
